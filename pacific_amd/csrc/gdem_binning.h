@@ -1,8 +1,6 @@
-// gdem_binning.h -- the count and scatter passes of the counting sort by
-// cell key (LinkedCell::LinkUpdate, Base/src/LinkedCell.cpp:1452-1547), as
-// device functions: the binning kernels call them, and the packed sphere
-// step runs them inside kernels whose other branch does the work of a step
-// without a rebuild.
+// gdem_binning.h -- the passes of the counting sort by cell key
+// (LinkedCell::LinkUpdate, Base/src/LinkedCell.cpp:1452-1547), as device
+// functions shared by the binning kernels and the rebuild of the packed step.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -79,6 +77,33 @@ __device__ __forceinline__ void scatter_pass(const int32_t* key, const int32_t* 
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const int k = key[i];
     perm[local[k] + bsum[k / kScanCells] + slot[i]] = i;
+  }
+}
+
+// Orders the slots of cell c by previous slot and writes its entries of the
+// sorted single-precision copy of position + radius and of the ids.
+__device__ __forceinline__ void sort_cell(const int32_t* local, const int32_t* bsum, int32_t* perm,
+                                          int32_t* cell_start, const PosSrc& src,
+                                          float4* pos_sorted, int32_t* ids_sorted, int c,
+                                          int ncell, int n) {
+  int beg = local[c] + bsum[c / kScanCells];
+  int end = (c + 1 < ncell) ? local[c + 1] + bsum[(c + 1) / kScanCells] : n;
+  for (int a = beg + 1; a < end; ++a) {
+    int v = perm[a];
+    int b = a - 1;
+    while (b >= beg && perm[b] > v) {
+      perm[b + 1] = perm[b];
+      --b;
+    }
+    perm[b + 1] = v;
+  }
+  cell_start[c] = beg;
+  if (c == ncell - 1) cell_start[ncell] = n;
+  for (int u = beg; u < end; ++u) {
+    const int s = perm[u];
+    const double4 p = src.pos(s);
+    pos_sorted[u] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
+    if (ids_sorted) ids_sorted[u] = src.aux[s].id;
   }
 }
 

@@ -118,12 +118,22 @@ struct gdem_ctx {
   bool packed = false;
   Pack pk[2]{};
   PackConst pkc[2]{};
-  uint32_t* d_omask = nullptr;
+  float* pk_path[2] = {nullptr, nullptr};
+  StepWords* d_step = nullptr;
+  int2* d_screen = nullptr;      // screening lists (StepLists)
+  int32_t* d_screen_count = nullptr;
+  float* d_min_gap = nullptr;
+  uint32_t* d_omask = nullptr;   // contacts of many particles (k_pairs)
   uint32_t* d_imask = nullptr;
   PairRec* d_prec = nullptr;
-  int32_t* d_queue = nullptr;   // candidates that may touch (t * 32 + entry)
-  int32_t* d_qcount = nullptr;  // its length, reset by the integrator
-  int32_t* d_wsrc = nullptr;    // 1: the packed copy's world angular velocity is derived
+  int32_t* d_path_rows = nullptr;
+  StepWords* h_step = nullptr;   // pinned: progress read back after a batch of chunks
+  double chunk_yield = kChunkSteps;  // steps a chunk of the last call did on average
+  // captured chunks: [0] one rebuild offered per kChunkSteps steps, [1] one
+  // before every step
+  hipGraphExec_t chunk_exec[2] = {nullptr, nullptr};
+  double chunk_dt[2] = {0., 0.};
+  int64_t chunk_made[2] = {-1, -1};
   // history (memory) contact models: per-particle memory tables, one per
   // state copy; allocated once a memory model is set and particles exist
   bool has_memory = false;
@@ -167,6 +177,7 @@ struct gdem_ctx {
   } while (0)
 
 static int collect_errors(gdem_ctx* c);
+static int halve_skin(gdem_ctx* c, int32_t peak);
 static int adapt_skin(gdem_ctx* c);
 
 static int set_err(gdem_ctx* c, int code, int id0, int id1) {
@@ -293,24 +304,35 @@ static void free_pack(gdem_ctx* c) {
     c->pk[k] = Pack{};
     c->pkc[k] = PackConst{};
   }
-  (void)hipFree(c->d_omask); (void)hipFree(c->d_imask); (void)hipFree(c->d_prec);
-  (void)hipFree(c->d_queue); (void)hipFree(c->d_qcount); (void)hipFree(c->d_wsrc);
+  for (float*& p : c->pk_path) {
+    (void)hipFree(p);
+    p = nullptr;
+  }
+  (void)hipFree(c->d_step); (void)hipFree(c->d_omask); (void)hipFree(c->d_imask);
+  (void)hipFree(c->d_prec);
   c->d_omask = c->d_imask = nullptr;
   c->d_prec = nullptr;
-  c->d_queue = c->d_qcount = c->d_wsrc = nullptr;
+  (void)hipFree(c->d_screen); (void)hipFree(c->d_screen_count); (void)hipFree(c->d_min_gap);
+  c->d_screen = nullptr;
+  c->d_screen_count = nullptr;
+  c->d_min_gap = nullptr;
+  c->d_step = nullptr;
+  (void)hipFree(c->d_path_rows);
+  c->d_path_rows = nullptr;
   c->packed = false;
 }
 
-// Capacity of one segment of the pair queue: the out entries of the
-// screening workgroups that append to it (workgroups b = k mod kQueueSegs).
-static int64_t queue_seg(const gdem_ctx* c) {
-  const int64_t nblk = (std::max<int64_t>(c->n, 1) + 255) / 256;
-  const int64_t nblk8 = (nblk + 7) / 8 * 8;
-  return (nblk8 + kQueueSegs - 1) / kQueueSegs * 256 * kListCap;
+static float skin_limit(const gdem_ctx* c);
+static float gap_unit(const gdem_ctx* c);
+
+static StepLists step_lists(const gdem_ctx* c) {
+  return StepLists{c->d_out_list, c->d_in_list, c->d_out_count, c->d_in_count, c->d_screen,
+                   c->d_screen_count, c->d_min_gap, gap_unit(c),
+                   step_in_one((int32_t)c->n), c->d_step, c->d_path_rows};
 }
 
 // Buffers of the packed layout for the current particle count (allocated on
-// first use: about 2 KB per particle, most of it the pair records).
+// first use: about 0.8 KB per particle, half of it the screening lists).
 static int alloc_pack(gdem_ctx* c) {
   if (c->pk[0].A) return GDEM_OK;
   const size_t n = (size_t)std::max<int64_t>(c->n, 1);
@@ -324,17 +346,22 @@ static int alloc_pack(gdem_ctx* c) {
     HIP_TRY(hipMalloc(&c->pkc[k].mi, sizeof(double2) * n));
     HIP_TRY(hipMalloc(&c->pkc[k].aux, sizeof(Aux) * n));
   }
-  HIP_TRY(hipMalloc(&c->d_omask, sizeof(uint32_t) * n));
-  HIP_TRY(hipMalloc(&c->d_imask, sizeof(uint32_t) * n));
-  HIP_TRY(hipMalloc(&c->d_prec, sizeof(PairRec) * n * kListCap));
-  HIP_TRY(hipMemset(c->d_imask, 0, sizeof(uint32_t) * n));
-  // every out entry at most once per step: a segment holds the entries of
-  // the screening workgroups (256 particles) that append to it
-  HIP_TRY(hipMalloc(&c->d_queue, sizeof(int32_t) * (size_t)queue_seg(c) * kQueueSegs));
-  HIP_TRY(hipMalloc(&c->d_qcount, sizeof(int32_t) * kQueueSegs));
-  HIP_TRY(hipMemset(c->d_qcount, 0, sizeof(int32_t) * kQueueSegs));
-  HIP_TRY(hipMalloc(&c->d_wsrc, sizeof(int32_t)));
-  HIP_TRY(hipMemset(c->d_wsrc, 0, sizeof(int32_t)));
+  for (float*& p : c->pk_path) HIP_TRY(hipMalloc(&p, sizeof(float) * n));
+  HIP_TRY(hipMalloc(&c->d_step, sizeof(StepWords)));
+  // many particles screen the out entries and keep records and masks
+  const bool one = step_in_one((int32_t)c->n);
+  HIP_TRY(hipMalloc(&c->d_screen, sizeof(int2) * n * kListCap * (one ? 2 : 1)));
+  if (!one) {
+    HIP_TRY(hipMalloc(&c->d_omask, sizeof(uint32_t) * n));
+    HIP_TRY(hipMalloc(&c->d_imask, sizeof(uint32_t) * n));
+    HIP_TRY(hipMalloc(&c->d_prec, sizeof(PairRec) * n * kListCap));
+    HIP_TRY(hipMemset(c->d_imask, 0, sizeof(uint32_t) * n));
+  }
+  HIP_TRY(hipMalloc(&c->d_screen_count, sizeof(int32_t) * n));
+  HIP_TRY(hipMalloc(&c->d_min_gap, sizeof(float) * n));
+  HIP_TRY(hipMalloc(&c->d_path_rows,
+                    sizeof(int32_t) * kRowSegs * kRowPad * (kTouchRow + 1)));
+  if (!c->h_step) HIP_TRY(hipHostMalloc(&c->h_step, sizeof(StepWords), hipHostMallocDefault));
   return GDEM_OK;
 }
 
@@ -342,11 +369,10 @@ static int alloc_pack(gdem_ctx* c) {
 // call other than gdem_step reads and writes the canonical copies).
 static int ensure_canon(gdem_ctx* c) {
   if (!c->packed) return GDEM_OK;
-  launch_from_pack(c->pk[c->cur], c->pk[1 - c->cur], c->pkc[c->cur], c->buf[c->cur], c->d_wsrc,
-                   c->bins.perm, c->d_skin, c->cur, (int32_t)c->n, c->stream);
+  launch_from_pack(c->pk[c->cur], c->pkc[c->cur], c->buf[c->cur], c->d_path, c->pk_path[c->cur],
+                   c->d_step, c->d_skin, c->cur, (int32_t)c->n, c->stream);
   HIP_TRY(hipGetLastError());
   c->packed = false;
-  c->graph_gen++;
   return GDEM_OK;
 }
 
@@ -355,11 +381,11 @@ static int ensure_packed(gdem_ctx* c) {
   if (c->packed) return GDEM_OK;
   const int ra = alloc_pack(c);
   if (ra) return ra;
-  launch_to_pack(c->buf[c->cur], c->pk[c->cur], c->pkc[0], c->pkc[1], c->d_wsrc, (int32_t)c->n,
-                 c->stream);
+  const StepLists l = step_lists(c);
+  launch_to_pack(c->buf[c->cur], c->pk[c->cur], c->pkc[0], c->pkc[1], l, c->d_skin,
+                 c->pk_path[c->cur], c->d_path, c->cur, (int32_t)c->n, c->stream);
   HIP_TRY(hipGetLastError());
   c->packed = true;
-  c->graph_gen++;
   return GDEM_OK;
 }
 
@@ -411,6 +437,9 @@ extern "C" int gdem_destroy(gdem_ctx* c) {
   (void)hipFree(c->d_wall_shapes); (void)hipFree(c->d_wall_sc); (void)hipFree(c->d_traj);
   free_wall_loads(c);
   free_pack(c);
+  (void)hipHostFree(c->h_step);
+  for (auto& g : c->chunk_exec)
+    if (g) (void)hipGraphExecDestroy(g);
   for (auto& e : c->ev_pool) { (void)hipEventDestroy(e.start); (void)hipEventDestroy(e.stop); }
   for (auto& row : c->graph_exec)
     for (auto& g : row)
@@ -507,9 +536,9 @@ static int alloc_particles(gdem_ctx* c, int64_t n, bool convex) {
     const int rw = reset_skin_words(c);  // the first evaluation rebuilds
     if (rw) return rw;
   }
-  // contact counts per workgroup of the sphere kernels, statistics parts
-  // (two per workgroup: pairs, walls)
-  c->nblk_slots = (int32_t)((((nn + 255) / 256 + 7) / 8) * 8);
+  // contact counts per workgroup of the sphere kernels (64 particles at
+  // least), statistics parts (two per workgroup: pairs, walls)
+  c->nblk_slots = (int32_t)((((nn + 63) / 64 + 7) / 8) * 8);
   HIP_TRY(hipMalloc(&c->d_blk_contacts, sizeof(unsigned long long) * c->nblk_slots));
   HIP_TRY(hipMemset(c->d_blk_contacts, 0, sizeof(unsigned long long) * c->nblk_slots));
   HIP_TRY(hipMalloc(&c->d_stat_part, sizeof(StatPart) * 2 * (size_t)c->nblk_slots));
@@ -1020,57 +1049,26 @@ static void launch_convex_step(gdem_ctx* c, int mode, double dtv, double dtd, bo
                        c->stream);
 }
 
-// Kernels of one evaluation in the packed layout: gated binning, pair kernel
-// (candidate sweep on a rebuild), integrator kernel.
-static int pack_launches(gdem_ctx* c, int mode, double dtv, double dtd, bool write_ft) {
-  const int p = c->cur;
-  const SkinGate gate{c->d_skin, p, skin_limit(c)};
-  const PackConst& kin = c->pkc[p];
-  const PosSrc src{c->pk[p].A, kin.rr, kin.aux};
-  const int nblk = (int)((c->n + 255) / 256);
-  const int nblk8 = ((nblk + 7) / 8) * 8;
-  PairArgs pa{};
-  DetectArgs& d = pa.d;
-  d.pos = c->bins.pos;
-  d.ids = c->bins.ids;
-  d.margin = prefilter_margin(c->grid, d.sizef);
-  d.perm = c->bins.perm;
-  d.cell_start = c->bins.cell_start;
-  d.row_rank = c->d_row_rank;
-  d.grid = c->grid;
-  d.n = (int32_t)c->n;
-  d.lstride = (int32_t)c->n;
-  d.out_list = c->d_out_list;
-  d.out_count = c->d_out_count;
-  d.in_list = c->d_in_list;
-  d.in_count = c->d_in_count;
-  d.err = c->d_err;
-  d.nblk8 = nblk8;
-  d.skin = c->skin;
-  d.gate = gate;
-  pa.in = c->pk[p];
-  pa.other = c->pk[1 - p];
-  pa.wsrc = c->d_wsrc;
-  pa.kin = kin;
-  pa.omask = c->d_omask;
-  pa.imask = c->d_imask;
-  pa.rec = c->d_prec;
-  pa.models = c->d_models;
-  pa.model_stride = kMaxMaterials;
-  pa.contacts = c->d_blk_contacts;
-  pa.queue = c->d_queue;
-  pa.qcount = c->d_qcount;
-  pa.qseg = (int32_t)std::min<int64_t>(queue_seg(c), 0x7fffffff);
-  TimedLaunch* ev = c->timing ? next_event_pair(c, 1) : nullptr;
-  launch_pair(c->bins, src, c->d_skin, pa, c->stream, ev ? ev->start : nullptr,
-              ev ? ev->stop : nullptr);
-  HIP_TRY(hipGetLastError());
-  IntegArgs a{};
-  a.in = c->pk[p];
-  a.out = c->pk[1 - p];
-  a.wsrc = c->d_wsrc;
-  a.kin = kin;
-  a.kout = c->pkc[1 - p];
+// Unit of the gap bounds in the skin lists' entries: the largest gap the
+// sweep lists (the skin and the pre-filter's margin beyond) fits in 20 bits.
+static float gap_unit(const gdem_ctx* c) {
+  float sizef[3];
+  const double most = c->skin + 4. * (double)prefilter_margin(c->grid, sizef);
+  return (float)(most / 1048575.);
+}
+
+// Launch records of the packed step: the step kernel's and the sweep's.
+static void packed_args(const gdem_ctx* c, double dt, StepArgs& a, DetectArgs& d) {
+  const int blk = step_particles((int32_t)c->n);
+  a = StepArgs{};
+  a.pk0 = c->pk[0];
+  a.pk1 = c->pk[1];
+  a.kc0 = c->pkc[0];
+  a.kc1 = c->pkc[1];
+  a.path0 = c->pk_path[0];
+  a.path1 = c->pk_path[1];
+  a.w = c->d_step;
+  a.path_rows = c->d_path_rows;
   a.perm = c->bins.perm;
   a.grid = c->grid;
   for (int dd = 0; dd < 3; ++dd) a.gmax[dd] = c->grid.nc[dd] * c->grid.edge[dd] * (1. - 1e-12);
@@ -1078,37 +1076,150 @@ static int pack_launches(gdem_ctx* c, int mode, double dtv, double dtd, bool wri
   a.model_stride = kMaxMaterials;
   a.walls = c->d_walls;
   a.nwalls = c->nwalls;
-  a.n = (int32_t)c->n;
-  a.lstride = (int32_t)c->n;
+  a.n = a.lstride = (int32_t)c->n;
   for (int dd = 0; dd < 3; ++dd) a.gravity[dd] = c->cfg.gravity[dd];
-  a.dt_vel = dtv;
-  a.dt_disp = dtd;
+  a.dt_vel = 0.5 * dt;
+  a.dt_disp = dt;
   a.crust_min = c->crust_min;
   a.out_list = c->d_out_list;
   a.in_list = c->d_in_list;
-  a.in_count = c->d_in_count;
+  a.out_count = c->d_out_count;
+  a.screen = c->d_screen;
+  a.screen_count = c->d_screen_count;
+  a.min_gap = c->d_min_gap;
+  a.F = c->d_F;
+  a.T = c->d_T;
+  a.limit = skin_limit(c);
+  a.gap_unit = gap_unit(c);
+  a.err = c->d_err;
+  a.contacts = c->d_blk_contacts;
+  a.nblk8 = (int32_t)(((c->n + blk - 1) / blk + 7) / 8 * 8);
   a.omask = c->d_omask;
   a.imask = c->d_imask;
   a.rec = c->d_prec;
-  a.F = write_ft ? c->d_F : nullptr;
-  a.T = write_ft ? c->d_T : nullptr;
-  a.gate = gate;
-  a.words = c->d_skin;
-  a.path = c->d_path;
-  a.err = c->d_err;
-  a.contacts = c->d_blk_contacts;
-  a.nblk8 = nblk8;
-  a.qcount = c->d_qcount;
-  ev = c->timing ? next_event_pair(c, 0) : nullptr;
-  launch_integ(mode, a, c->stream, ev ? ev->start : nullptr, ev ? ev->stop : nullptr);
+  a.in_count = c->d_in_count;
+  d = DetectArgs{};
+  d.pos = c->bins.pos;
+  d.ids = c->bins.ids;
+  d.margin = prefilter_margin(c->grid, d.sizef);
+  d.perm = c->bins.perm;
+  d.cell_start = c->bins.cell_start;
+  d.row_rank = c->d_row_rank;
+  d.grid = c->grid;
+  d.n = d.lstride = (int32_t)c->n;
+  d.out_list = c->d_out_list;
+  d.out_count = c->d_out_count;
+  d.in_list = c->d_in_list;
+  d.in_count = c->d_in_count;
+  d.err = c->d_err;
+  d.nblk8 = (int32_t)(((c->n + 255) / 256 + 7) / 8 * 8);
+  d.skin = c->skin;
+  d.gap_unit = a.gap_unit;
+  d.gate = SkinGate{nullptr, 0, a.limit, c->d_step};
+}
+
+// One chunk: a gated rebuild, then `steps` step kernels (at most
+// kChunkSteps).
+static int chunk_launches(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, int steps) {
+  const PosSrc s0{c->pk[0].A, c->pkc[0].rr, c->pkc[0].aux};
+  const PosSrc s1{c->pk[1].A, c->pkc[1].rr, c->pkc[1].aux};
+  launch_pack_rebuild(c->bins, s0, s1, c->d_step, c->d_skin, d, step_lists(c), c->pk[0],
+                      c->pk[1], c->stream);
   HIP_TRY(hipGetLastError());
+  for (int j = 0; j < steps; ++j) {
+    hipEvent_t e[4] = {nullptr, nullptr, nullptr, nullptr};
+    for (int k = 0; c->timing && k < (step_in_one((int32_t)c->n) ? 1 : 2); ++k)
+      if (TimedLaunch* ev = next_event_pair(c, k)) {
+        e[2 * k] = ev->start;
+        e[2 * k + 1] = ev->stop;
+      }
+    launch_step(a, j, j + 1 == steps ? kChunkSteps : j + 1, j == 0, c->stream, e[0], e[1], e[2],
+                e[3]);
+    HIP_TRY(hipGetLastError());
+  }
+  return GDEM_OK;
+}
+
+// kChunkSteps steps as one graph, captured on first use: one chunk (each =
+// false) or a chunk per step.
+static int chunk_graph(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, bool each, double dt) {
+  const int k = each ? 1 : 0;
+  hipGraphExec_t& ge = c->chunk_exec[k];
+  if (!ge || c->chunk_dt[k] != dt || c->chunk_made[k] != c->graph_gen) {
+    if (ge) {
+      HIP_TRY(hipGraphExecDestroy(ge));
+      ge = nullptr;
+    }
+    HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+    int rc = GDEM_OK;
+    if (!each) rc = chunk_launches(c, a, d, kChunkSteps);
+    else
+      for (int j = 0; j < kChunkSteps && rc == GDEM_OK; ++j) rc = chunk_launches(c, a, d, 1);
+    hipGraph_t graph = nullptr;
+    const hipError_t e = hipStreamEndCapture(c->stream, &graph);
+    if (rc) {
+      if (graph) (void)hipGraphDestroy(graph);
+      return rc;
+    }
+    HIP_TRY(e);
+    const hipError_t ei = hipGraphInstantiate(&ge, graph, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(graph);
+    HIP_TRY(ei);
+    c->chunk_dt[k] = dt;
+    c->chunk_made[k] = c->graph_gen;
+  }
+  HIP_TRY(hipGraphLaunch(ge, c->stream));
+  return GDEM_OK;
+}
+
+// n steps in the packed layout after launch_move_pack.  A chunk does
+// kChunkSteps steps unless a rebuild falls into it, so the host launches the
+// chunks it expects to need, reads the progress and launches the rest; every
+// chunk does at least one step.  With the occupancy check off the call must
+// not wait for the stream: a rebuild is then offered before every step.
+static int packed_steps(gdem_ctx* c, int32_t n, double dt) {
+  StepArgs a;
+  DetectArgs d;
+  packed_args(c, dt, a, d);
+  const bool graph = c->use_graph && !c->timing;
+  int rc = GDEM_OK;
+  if (!c->skin_adapt || c->timing) {
+    for (int32_t k = 0; k < n && rc == GDEM_OK;) {
+      const bool run = graph && n - k >= kChunkSteps;
+      rc = run ? chunk_graph(c, a, d, true, dt) : chunk_launches(c, a, d, 1);
+      k += run ? kChunkSteps : 1;
+    }
+  } else {
+    for (int32_t done = 0; done < n && rc == GDEM_OK;) {
+      int32_t left = n - done;
+      if (left < kChunkSteps) {
+        rc = chunk_launches(c, a, d, left);
+      } else {
+        const int32_t chunks = std::max(1, (int32_t)((double)left / c->chunk_yield + 0.5));
+        for (int32_t k = 0; k < chunks && rc == GDEM_OK; ++k)
+          rc = graph ? chunk_graph(c, a, d, false, dt) : chunk_launches(c, a, d, kChunkSteps);
+      }
+      if (rc) break;
+      HIP_TRY(hipMemcpyAsync(c->h_step, c->d_step, sizeof(StepWords), hipMemcpyDeviceToHost,
+                             c->stream));
+      HIP_TRY(hipStreamSynchronize(c->stream));
+      done = c->h_step->slot[kChunkSteps].done;
+    }
+    if (rc == GDEM_OK && n >= kChunkSteps)
+      c->chunk_yield = std::min<double>(
+          kChunkSteps, std::max(1., (double)n / (double)std::max(c->h_step->chunks, 1)));
+  }
+  if (rc) return rc;
+  for (int32_t k = 0; k < n; ++k) c->time += dt;
+  if (n & 1) c->cur = 1 - c->cur;
+  c->binned = false;
+  c->force_evals += n;
   return GDEM_OK;
 }
 
 // Kernels of one force evaluation on the current copy (binning first when
 // positions changed); no host bookkeeping, so the sequence can be captured.
 static int force_launches(gdem_ctx* c, int mode, double dtv, double dtd, bool write_ft) {
-  if (c->packed) return pack_launches(c, mode, dtv, dtd, write_ft);
   const bool skin = !c->convex && c->skin > 0.;
   const SkinGate gate = skin ? SkinGate{c->d_skin, c->cur, skin_limit(c)} : SkinGate{};
   if (skin) {
@@ -1152,6 +1263,7 @@ static int force_launches(gdem_ctx* c, int mode, double dtv, double dtd, bool wr
     d.err = c->d_err;
     d.nblk8 = nblk8;
     d.skin = skin ? c->skin : 0.;
+    d.gap_unit = skin ? gap_unit(c) : 0.f;
     d.gate = gate;
     ForceArgs a{};
     a.in = c->buf[c->cur];
@@ -1457,13 +1569,15 @@ extern "C" int gdem_step(gdem_ctx* c, int32_t nsteps, double dt) {
     if (rc) return rc;
     note_move_step(c, dt);
     launch_move_pack(c->pk[c->cur], c->pkc[c->cur], c->d_F, c->d_T, (int32_t)c->n, c->grid,
-                     0.5 * dt, dt, c->d_err, SkinGate{c->d_skin, c->cur, skin_limit(c)},
-                     c->d_path, c->d_wsrc, c->stream);
+                     0.5 * dt, dt, c->d_err, skin_limit(c), c->pk_path[c->cur], c->d_step,
+                     c->d_path_rows, c->cur, nsteps, c->stream);
     HIP_TRY(hipGetLastError());
-  } else {
-    rc = gdem_move(c, 0.5 * dt, dt);
+    rc = packed_steps(c, nsteps, dt);
     if (rc) return rc;
+    return c->skin_adapt && !c->timing ? halve_skin(c, c->h_step->peak) : adapt_skin(c);
   }
+  rc = gdem_move(c, 0.5 * dt, dt);
+  if (rc) return rc;
   if (c->kin.any_live()) return moving_wall_steps(c, nsteps, dt);
   const bool graph = c->use_graph && !c->timing && c->rec_cap == 0;
   for (int32_t k = 0; k < nsteps;) {
@@ -1494,21 +1608,25 @@ static int list_peak(gdem_ctx* c, int32_t* peak) {
 }
 
 // Degrade before the skin lists overflow: when the last list build left a
-// particle within kListHeadroom entries of the capacity, halve the skin (the
-// lists then hold fewer candidates; below 5 % of the largest radius the skin
-// is switched off and lists hold contacts only) and rebuild at the next
-// evaluation.  The physics does not depend on the skin.
-static int adapt_skin(gdem_ctx* c) {
-  if (!c->skin_adapt || !(c->skin > 0.) || c->convex) return GDEM_OK;
-  int32_t peak = 0;
-  int rc = list_peak(c, &peak);
-  if (rc) return rc;
+// particle within kListHeadroom entries of the capacity (peak: its longest
+// list), halve the skin (the lists then hold fewer candidates; below 5 % of
+// the largest radius the skin is switched off and lists hold contacts only)
+// and rebuild at the next evaluation.  The physics does not depend on the
+// skin.
+static int halve_skin(gdem_ctx* c, int32_t peak) {
   if (peak <= kListCap - kListHeadroom) return GDEM_OK;
   // a list that overflowed has raised GDEM_ERR_CAPACITY: report it
-  rc = collect_errors(c);
+  const int rc = collect_errors(c);
   if (rc) return rc;
   c->skin_halvings++;
   return gdem_set_skin(c, 0.5 * c->skin);
+}
+
+static int adapt_skin(gdem_ctx* c) {
+  if (!c->skin_adapt || !(c->skin > 0.) || c->convex) return GDEM_OK;
+  int32_t peak = 0;
+  const int rc = list_peak(c, &peak);
+  return rc ? rc : halve_skin(c, peak);
 }
 
 extern "C" int gdem_set_skin_adapt(gdem_ctx* c, int32_t on) {

@@ -67,25 +67,48 @@ constexpr unsigned long long kNoErr = ~0ull;
 // the next evaluation:
 //   * the evaluation reading copy p rebuilds when need[p] is set; its first
 //     kernel clears need[1-p] and counts the rebuild; its integrator tail
-//     (path restarted on a rebuild) raises need[1-p] and one thread writes
-//     rebuilt[1-p];
+//     (path restarted on a rebuild) raises need[1-p];
 //   * a stand-alone move in place of copy p raises need[p].
 // No kernel of an evaluation writes a word it reads, and the need words are
-// written only by the few particles that cross the limit (integer OR).
+// written only by the few particles that cross the limit (integer OR).  The
+// packed step keeps its own words (StepWords) and hands them over when the
+// layout changes.
 struct SkinWords {
   int32_t need[2];
-  int32_t rebuilt[2];  // rebuilt[p]: the evaluation that wrote copy p rebuilt
   int32_t rebuilds;
 };
 
-// Rebuild decision of the evaluation reading copy p (the same in every
-// kernel of that evaluation); w == nullptr: no skin lists, the lists are
-// rebuilt at every evaluation.
+// Progress of the packed step sequence of one gdem_step call.  The launches
+// of a chunk are numbered: launch j reads slot j and writes slot j + 1, the
+// last one writes slot kChunkSteps, which the next chunk's rebuild kernels
+// read and copy to slot 0.  A slot holds the steps done so far, the copy the
+// next step reads, whether a rebuild is due before it, whether the last step
+// was a rebuild and whether the copy holds the world angular velocities.  A launch that finds a rebuild due (and none offered
+// right before it) or the target reached passes its slot on and does nothing
+// else, so the host may launch chunks without knowing where rebuilds fall.
+constexpr int kChunkSteps = 16;
+struct StepSlot {
+  int32_t done, cur, need, rebuilt, wstored;
+};
+struct StepWords {
+  StepSlot slot[kChunkSteps + 1];
+  int32_t target;  // steps of this call
+  int32_t peak;    // longest list of the last build, if near the capacity
+  int32_t chunks;  // chunks that found steps to do
+};
+
+// Rebuild decision: of the evaluation reading copy p (the same in every
+// kernel of that evaluation), or with sw of the chunk (slot 0); neither: no
+// skin lists, the lists are rebuilt at every evaluation.
 struct SkinGate {
   const SkinWords* w;
   int32_t p;
   float limit;  // skin / 2, rounded down
-  __device__ __forceinline__ bool rebuild() const { return !w || w->need[p] != 0; }
+  const StepWords* sw;  // null: w and p decide
+  __device__ __forceinline__ bool rebuild() const {
+    if (sw) return sw->slot[0].need != 0 && sw->slot[0].done < sw->target;
+    return !w || w->need[p] != 0;
+  }
 };
 
 // Path length of a particle after a drift of length depl, restarted when the
@@ -113,9 +136,10 @@ struct PosSrc {
 
 // A contact-list entry: partner slot and a code packing the periodic shift to
 // apply to the partner ((s+1) in 2 bits per axis), whether this particle is
-// the first body of the pair (bit 6) and, in bits 7-11, the position of the
-// mirror entry in the partner's other list (an out entry holds its index in
-// the partner's in-list, an in entry its index in the partner's out-list).
+// the first body of the pair (bit 6) and, in the skin lists, the position of
+// the mirror entry in the partner's other list (bits 7-11) and a lower bound
+// of the pair's gap when the list was built, in units of gap_unit (bits
+// 12-31).
 struct DetectArgs {
   const float4* pos;      // single-precision positions + radius, sorted order
   const int32_t* ids;     // particle ids, sorted order (skin lists)
@@ -140,6 +164,7 @@ struct DetectArgs {
   // the few within the pre-filter margin beyond) instead of contacts; the
   // sweep runs only when the gate says a rebuild is due
   double skin;
+  float gap_unit;  // unit of the entries' gap bounds
   SkinGate gate;
 };
 
@@ -370,13 +395,10 @@ void launch_keys(const State& s, int32_t n, const Grid& g, const int32_t* row_ra
 void launch_binning(Bins& b, const PosSrc& src, int32_t n, const Grid& g, const int32_t* row_rank,
                     unsigned long long* err, hipStream_t st, SkinGate gate = SkinGate{},
                     SkinWords* words = nullptr, int32_t* in_count = nullptr);
-// The scan and the per-cell sort of a gated binning alone (the count and
-// scatter passes then run elsewhere: gdem_binning.h).
+// The scan of a gated binning alone.
 void launch_scan(const Bins& b, int32_t ncell, SkinGate gate, hipStream_t st);
 void launch_list_peak(const int32_t* out, const int32_t* in, int32_t n, int32_t* peak,
                       hipStream_t st);
-void launch_cellsort(const Bins& b, const PosSrc& src, int32_t ncell, int32_t n, SkinGate gate,
-                     hipStream_t st);
 void launch_detect(const DetectArgs& a, hipStream_t st);
 // With events, they record the kernel's own start and end (timing).  memory:
 // the history-model variant (a.hin / a.hout used).
@@ -419,8 +441,8 @@ void launch_set_state(const State& s, double4* F, double4* T, int32_t n, const d
 struct Pack {
   double4* A;  // x, y, z, q.x
   double4* B;  // v, q.y
-  double4* C;  // world angular velocity (.w unused), stored only when the
-               // W word (wsrc) is 0; otherwise derived (world_omega)
+  double4* C;  // world angular velocity (.w unused); where a step has not
+               // stored it (StepSlot::wstored), derived (world_omega)
   double4* D;  // body-frame angular velocity, q.z
   double* E;   // q.w
 };
@@ -438,31 +460,40 @@ struct PairRec {
   double f[3], ta[3], tb[3];
 };
 
-// Segments of the pair queue (workgroup b of the screening appends to
-// segment b mod kQueueSegs).
-constexpr int kQueueSegs = 64;
-
-struct PairArgs {
-  DetectArgs d;        // the candidate sweep of a rebuild (d.in unused)
-  Pack in;
-  Pack other;          // the other copy: the orientations before the last step
-  int32_t* wsrc;       // W word: 1 when in.C is not stored (world_omega)
-  PackConst kin;
-  uint32_t* omask;     // [n] out entries in contact (cleared by the screening)
-  uint32_t* imask;     // [n] in entries in contact (atomic OR, zero on entry)
-  PairRec* rec;
-  const Model* models;
-  int32_t model_stride;
-  unsigned long long* contacts;  // contact counts, one per workgroup (added to)
-  int32_t* queue;      // candidates that may touch, t * 32 + entry, in segments
-  int32_t* qcount;     // [kQueueSegs] segment lengths (zero on entry)
-  int32_t qseg;        // capacity of one segment
+// The candidate lists and what the packed step makes of them: the screening
+// lists [2 kListCap][n] (out entries only: [kListCap][n]) by increasing gap
+// bound, their lengths, each particle's smallest gap bound.
+struct StepLists {
+  const int2* out_list;
+  int2* in_list;  // put in the order of summation
+  const int32_t* out_count;
+  const int32_t* in_count;
+  int2* screen;
+  int32_t* screen_count;
+  float* min_gap;
+  float gap_unit;
+  bool both;  // out and in entries (k_step), or out entries (k_pairs)
+  StepWords* words;
+  int32_t* path_rows;  // as StepArgs
 };
 
-struct IntegArgs {
-  Pack in, out;
-  int32_t* wsrc;       // W word, set for the copy this kernel writes
-  PackConst kin, kout;
+// Counters of one launch that many workgroups add to: kRowSegs segments
+// (workgroup b uses segment b mod kRowSegs), kRowPad words apart.
+constexpr int kRowSegs = 64;
+constexpr int kRowPad = 32;
+constexpr int kTouchRow = kChunkSteps + 1;
+
+// Launch record of the packed step.  The kernels take the copy they read from
+// the step words, so one record (and one captured graph) serves every step.
+struct StepArgs {
+  Pack pk0, pk1;
+  PackConst kc0, kc1;
+  float *path0, *path1;  // path lengths since the last rebuild, slot order
+  StepWords* w;
+  // rows 0..kChunkSteps: the largest path length before launch j (bits of a
+  // float; row kChunkSteps is handed over as the slot is); row kTouchRow: the
+  // touching candidates of the last build
+  int32_t* path_rows;
   const int32_t* perm;
   Grid grid;
   double gmax[3];      // below nc * edge by a relative 1e-12: surely inside the grid
@@ -476,40 +507,55 @@ struct IntegArgs {
   double crust_min;    // smallest crust: a drift below it raises no MotionError
   const int2* out_list;
   const int2* in_list;
-  const int32_t* in_count;
-  const uint32_t* omask;
-  uint32_t* imask;     // cleared after reading
-  const PairRec* rec;
-  double4* F;          // written when non-null
+  const int32_t* out_count;
+  const int2* screen;  // screening lists (StepLists)
+  const int32_t* screen_count;
+  const float* min_gap;
+  double4* F;          // written by the last step
   double4* T;
-  SkinGate gate;
-  SkinWords* words;
-  float* path;         // path length since the last rebuild, slot order
+  float limit;         // skin / 2, rounded down
+  float gap_unit;
   unsigned long long* err;
-  unsigned long long* contacts;  // per workgroup (walls)
-  int32_t nblk8;
-  int32_t* qcount;     // the pair queue's segment lengths, cleared for the next step
+  unsigned long long* contacts;  // per workgroup
+  int32_t nblk8;       // workgroups of step_particles(n) particles, a multiple of 8
+  // many particles (k_pairs, k_integ): records and masks of the contacts
+  uint32_t* omask;     // out entries in contact
+  uint32_t* imask;     // in entries in contact (integer OR; cleared after reading)
+  PairRec* rec;
+  const int32_t* in_count;
 };
 
-// Both conversions keep the W word: to_pack stores the world angular
-// velocity (word 0); from_pack derives it where it is not stored, from the
-// other copy (other) at the slots perm gives when the last evaluation was a
-// rebuild (words->rebuilt[p]).
+// Both conversions move the state, the path lengths and the need word of
+// copy p.
 void launch_to_pack(const State& s, const Pack& pk, const PackConst& k0, const PackConst& k1,
-                    int32_t* wsrc, int32_t n, hipStream_t st);
-void launch_from_pack(const Pack& pk, const Pack& other, const PackConst& k, const State& s,
-                      const int32_t* wsrc, const int32_t* perm, const SkinWords* words, int p,
-                      int32_t n, hipStream_t st);
-// The pair stage of a packed step, the binning of a rebuild included (its
-// count and scatter passes run inside the pair kernels).
-void launch_pair(const Bins& b, const PosSrc& src, SkinWords* words, const PairArgs& a,
-                 hipStream_t st, hipEvent_t start = nullptr, hipEvent_t stop = nullptr);
-void launch_integ(int mode, const IntegArgs& a, hipStream_t st, hipEvent_t start = nullptr,
-                  hipEvent_t stop = nullptr);
-// Kick + drift of the packed copy in place (the opening half of gdem_step).
+                    const StepLists& l, const SkinWords* words, float* path, const float* path_in,
+                    int p, int32_t n, hipStream_t st);
+void launch_from_pack(const Pack& pk, const PackConst& k, const State& s, float* path_out,
+                      const float* path, const StepWords* w, SkinWords* words, int p, int32_t n,
+                      hipStream_t st);
+// The gated rebuild that opens a chunk.
+void launch_pack_rebuild(const Bins& b, const PosSrc& src0, const PosSrc& src1, StepWords* w,
+                         SkinWords* words, const DetectArgs& d, const StepLists& l,
+                         const Pack& pk0, const Pack& pk1, hipStream_t st);
+// Fewer than kStepSmall particles step in one kernel, more in two; particles
+// per workgroup of the integrating kernel; largest number of particles per
+// lane of k_pairs, and the workgroups it keeps at least.
+constexpr int kStepSmall = 524288;
+constexpr int kPairPer = 6;
+constexpr int kPairGrid = 640;
+bool step_in_one(int32_t n);
+int step_particles(int32_t n);
+// One step (launch j_in of a chunk, handing over to slot j_out); after: a
+// rebuild was offered right before it.  With events, start and stop record the
+// integrating kernel's own start and end, start1 and stop1 those of k_pairs.
+void launch_step(const StepArgs& a, int j_in, int j_out, bool after, hipStream_t st,
+                 hipEvent_t start = nullptr, hipEvent_t stop = nullptr,
+                 hipEvent_t start1 = nullptr, hipEvent_t stop1 = nullptr);
+// Kick + drift of the packed copy p in place (the opening half of gdem_step)
+// and the start of a sequence of nsteps steps.
 void launch_move_pack(const Pack& pk, const PackConst& k, const double4* F, const double4* T,
                       int32_t n, const Grid& g, double dt_vel, double dt_disp,
-                      unsigned long long* err, SkinGate gate, float* path, int32_t* wsrc,
-                      hipStream_t st);
+                      unsigned long long* err, float limit, float* path, StepWords* w,
+                      int32_t* path_rows, int p, int32_t nsteps, hipStream_t st);
 
 }  // namespace gdem

@@ -151,32 +151,6 @@ __global__ void __launch_bounds__(kBlock) k_scatter(const int32_t* key, const in
   scatter_pass(key, slot, local, bsum, perm, n);
 }
 
-// One cell of k_cellsort.
-__device__ __forceinline__ void sort_cell(const int32_t* local, const int32_t* bsum, int32_t* perm,
-                                          int32_t* cell_start, const PosSrc& src,
-                                          float4* pos_sorted, int32_t* ids_sorted, int c,
-                                          int ncell, int n) {
-  int beg = local[c] + bsum[c / kScanCells];
-  int end = (c + 1 < ncell) ? local[c + 1] + bsum[(c + 1) / kScanCells] : n;
-  for (int a = beg + 1; a < end; ++a) {
-    int v = perm[a];
-    int b = a - 1;
-    while (b >= beg && perm[b] > v) {
-      perm[b + 1] = perm[b];
-      --b;
-    }
-    perm[b + 1] = v;
-  }
-  cell_start[c] = beg;
-  if (c == ncell - 1) cell_start[ncell] = n;
-  for (int u = beg; u < end; ++u) {
-    const int s = perm[u];
-    const double4 p = src.pos(s);
-    pos_sorted[u] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
-    if (ids_sorted) ids_sorted[u] = src.aux[s].id;
-  }
-}
-
 // Orders each cell by previous slot, which makes the permutation independent of
 // the order in which the count pass's atomics were served, then writes the
 // cell's entries of the sorted single-precision copy of position + radius
@@ -233,7 +207,6 @@ __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a) {
       a.path[t] = len;
       if (len > a.gate.limit) atomicOr(&a.words->need[1 - a.gate.p], 1);
     }
-    if (t == 0) a.words->rebuilt[1 - a.gate.p] = rebuilt ? 1 : 0;
   }
   // contact counter: wave sum, then one integer atomic per workgroup
   unsigned long long c = (unsigned long long)ncont;
@@ -476,8 +449,6 @@ void launch_binning(Bins& b, const PosSrc& src, int32_t n, const Grid& g, const 
                      gate);
 }
 
-// The scan and the per-cell sort of a gated binning, for launch sequences
-// that run the count and scatter passes inside kernels of their own.
 // Largest list length of any particle (its outgoing or incoming entries at
 // the last list build): a fixed-size tree per workgroup, then one atomic.
 __global__ void __launch_bounds__(256) k_list_peak(const int32_t* out, const int32_t* in, int32_t n,
@@ -506,13 +477,6 @@ void launch_scan(const Bins& b, int32_t ncell, SkinGate gate, hipStream_t st) {
   const int nb = nblocks(ncell, kScanCells);
   hipLaunchKernelGGL(k_scan, dim3(nb), dim3(kScanBlock), 0, st, b.cnt, b.local, b.bsum, b.ticket,
                      ncell, nb, gate);
-}
-
-void launch_cellsort(const Bins& b, const PosSrc& src, int32_t ncell, int32_t n, SkinGate gate,
-                     hipStream_t st) {
-  hipLaunchKernelGGL(k_cellsort, dim3(std::min(nblocks(ncell, kBlock), kGateGrid)), dim3(kBlock),
-                     0, st, b.local, b.bsum, b.perm, b.cell_start, src, b.pos, b.ids, ncell, n,
-                     gate);
 }
 
 void launch_wall_loads(const ForceArgs& a, double4* part, double4* out, hipStream_t st) {

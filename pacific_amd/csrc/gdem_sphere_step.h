@@ -30,16 +30,14 @@ struct Detector {
   // Appends partner u (entry code) to this particle's out-list and the
   // mirror entry to u's in-list; id and id2 name the two in a capacity error.
   __device__ __forceinline__ void append(int u, int code, int32_t id, int32_t id2) {
-    // each entry also records where its mirror sits in the partner's other
-    // list (bits 7-11; an index at or beyond the capacity is never used)
     const int kin = atomicAdd(&a.in_count[u], 1);
     if (nout < kListCap) {
-      a.out_list[(size_t)nout * a.lstride + t] = make_int2(u, code | (min(kin, 31) << 7));
+      a.out_list[(size_t)nout * a.lstride + t] = make_int2(u, code);
     } else {
       atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)id);
     }
     if (kin < kListCap) {
-      a.in_list[(size_t)kin * a.lstride + u] = make_int2(t, mirror_code(code) | (min(nout, 31) << 7));
+      a.in_list[(size_t)kin * a.lstride + u] = make_int2(t, mirror_code(code));
     } else {
       atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)id2);
     }
@@ -56,14 +54,16 @@ struct Detector {
     const float dyf = (p2f.y + sy * a.sizef[1]) - mef.y;
     const float dzf = (p2f.z + sz * a.sizef[2]) - mef.z;
     const float rsf = mef.w + p2f.w + (float)a.skin + a.margin;
-    if (dxf * dxf + dyf * dyf + dzf * dzf > rsf * rsf) return;
+    const float d2f = dxf * dxf + dyf * dyf + dzf * dzf;
+    if (d2f > rsf * rsf) return;
     if (a.skin > 0.) {
       // candidate: the pre-filter alone decides (every pair with gap below
       // the skin passes it, and the few within the margin beyond); the
       // contact test of every step is made on the candidates with the same
       // body order.  The in-list positions are taken afterwards (link()).
       const int32_t id = a.ids[t];
-      const int code = pack_code(sx, sy, sz, same ? (id < a.ids[u]) : true);
+      const int code = pack_code(sx, sy, sz, same ? (id < a.ids[u]) : true) |
+                       pack_gap(sqrtf(d2f) - (mef.w + p2f.w) - a.margin, a.gap_unit);
       if (nout < kListCap) a.out_list[(size_t)nout * a.lstride + t] = make_int2(u, code);
       else atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)id);
       ++nout;
@@ -103,10 +103,10 @@ struct Detector {
     append(u, pack_code(sx, sy, sz, first), ax.id, ax2.id);
   }
 
-  // Skin lists: the in-list position of every out entry the sweep stored
-  // (partner and code), from integer atomics issued four at a time, written
-  // into the entry (bits 7-11) and with the mirror entry into the partner's
-  // in-list.
+  // Skin lists: the mirror of every out entry the sweep stored, into the
+  // partner's in-list, at positions from integer atomics issued four at a
+  // time.  Each entry also records where its mirror sits in the partner's
+  // other list (bits 7-11; an index at or beyond the capacity is never used).
   __device__ __forceinline__ void link() {
     const int n = min(nout, kListCap);
     for (int e0 = 0; e0 < n; e0 += 4) {
@@ -124,7 +124,8 @@ struct Detector {
         const int e = e0 + k, u = en[k].x, code = en[k].y;
         a.out_list[(size_t)e * a.lstride + t] = make_int2(u, code | (min(kin[k], 31) << 7));
         if (kin[k] < kListCap)
-          a.in_list[(size_t)kin[k] * a.lstride + u] = make_int2(t, mirror_code(code) | (e << 7));
+          a.in_list[(size_t)kin[k] * a.lstride + u] =
+              make_int2(t, mirror_code(code) | (e << 7) | (int)((uint32_t)code & kGapMask));
         else
           atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)a.ids[u]);
       }

@@ -21,6 +21,19 @@ __device__ __forceinline__ int mirror_code(int code) {
   return pack_code(1 - (code & 3), 1 - ((code >> 2) & 3), 1 - ((code >> 4) & 3), !(code & 64));
 }
 
+// Lower bound of a pair's gap (m, negative: 0) in the upper 20 bits of an
+// entry's code, and the bound an entry carries: both round down (a relative
+// 1e-6 covers the single-precision product and quotient).
+constexpr uint32_t kGapMask = 0xfffff000u;
+constexpr float kGapSteps = 1048575.f;
+__device__ __forceinline__ int pack_gap(float gap, float unit) {
+  const float q = fminf(fmaxf(gap, 0.f) / unit, kGapSteps);
+  return (int)((uint32_t)q << 12);
+}
+__device__ __forceinline__ float gap_bound(int code, float unit) {
+  return (float)((uint32_t)code >> 12) * unit * 0.999999f;
+}
+
 // Cell::GetCell (Base/src/Cell.cpp:172-184); periodic indices are clamped to
 // the grid after the wrap of the position.  Returns false outside the grid.
 __device__ __forceinline__ bool cell_of(const Grid& g, v3 x, int* ijk) {
