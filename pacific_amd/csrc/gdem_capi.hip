@@ -97,6 +97,7 @@ struct gdem_ctx {
   uint32_t* d_mask = nullptr;
   int32_t* d_work = nullptr;
   int32_t* d_nwork = nullptr;
+  int32_t* d_near = nullptr;
   CShape h_wall_shapes[kMaxWalls]{};
   double4 h_wall_sc[kMaxWalls]{};
   CShape* d_wall_shapes = nullptr;
@@ -431,7 +432,7 @@ extern "C" int gdem_destroy(gdem_ctx* c) {
   free_cstate(c->cbuf[0]);
   free_cstate(c->cbuf[1]);
   (void)hipFree(c->d_cand); (void)hipFree(c->d_crec); (void)hipFree(c->d_mask); (void)hipFree(c->d_work);
-  (void)hipFree(c->d_nwork); (void)hipFree(c->d_shapes);
+  (void)hipFree(c->d_nwork); (void)hipFree(c->d_near); (void)hipFree(c->d_shapes);
   (void)hipFree(c->d_skin); (void)hipFree(c->d_cmask); (void)hipFree(c->d_path);
   (void)hipFree(c->d_blk_contacts); (void)hipFree(c->d_stats); (void)hipFree(c->d_stat_part);
   (void)hipFree(c->d_wall_shapes); (void)hipFree(c->d_wall_sc); (void)hipFree(c->d_traj);
@@ -489,7 +490,7 @@ static int alloc_particles(gdem_ctx* c, int64_t n, bool convex) {
   (void)hipFree(c->d_out_list); (void)hipFree(c->d_in_list); (void)hipFree(c->d_out_count); (void)hipFree(c->d_in_count);
   (void)hipFree(c->d_rec); (void)hipFree(c->d_rec_count);
   (void)hipFree(c->d_cand); (void)hipFree(c->d_crec); (void)hipFree(c->d_mask); (void)hipFree(c->d_work);
-  (void)hipFree(c->d_nwork);
+  (void)hipFree(c->d_nwork); (void)hipFree(c->d_near);
   (void)hipFree(c->d_skin); (void)hipFree(c->d_cmask); (void)hipFree(c->d_path);
   (void)hipFree(c->d_blk_contacts); (void)hipFree(c->d_stat_part);
   free_history(c);
@@ -513,6 +514,7 @@ static int alloc_particles(gdem_ctx* c, int64_t n, bool convex) {
   c->d_mask = nullptr;
   c->d_work = nullptr;
   c->d_nwork = nullptr;
+  c->d_near = nullptr;
   c->n = n;
   c->convex = convex;
   c->rmax = 0.;
@@ -525,8 +527,9 @@ static int alloc_particles(gdem_ctx* c, int64_t n, bool convex) {
     HIP_TRY(hipMalloc(&c->d_crec, sizeof(CRec) * nn * kCandCap));
     HIP_TRY(hipMalloc(&c->d_mask, sizeof(uint32_t) * nn));
     HIP_TRY(hipMalloc(&c->d_work, sizeof(int32_t) * nn * kCandCap));
-    HIP_TRY(hipMalloc(&c->d_nwork, sizeof(int32_t)));
-    HIP_TRY(hipMemset(c->d_nwork, 0, sizeof(int32_t)));
+    HIP_TRY(hipMalloc(&c->d_near, sizeof(int32_t) * nn * kCandCap));
+    HIP_TRY(hipMalloc(&c->d_nwork, sizeof(int32_t) * 2));
+    HIP_TRY(hipMemset(c->d_nwork, 0, sizeof(int32_t) * 2));
   } else {
     HIP_TRY(hipMalloc(&c->d_out_list, sizeof(int2) * nn * kListCap));
     HIP_TRY(hipMalloc(&c->d_skin, sizeof(SkinWords)));
@@ -998,6 +1001,8 @@ static void launch_convex_step(gdem_ctx* c, int mode, double dtv, double dtd, bo
   g.cand = c->d_cand;
   g.work = c->d_work;
   g.nwork = c->d_nwork;
+  g.near = c->d_near;
+  g.nnear = c->d_nwork + 1;
   g.walls = c->d_walls;
   g.wall_shapes = c->d_wall_shapes;
   g.wall_sc = c->d_wall_sc;

@@ -3,7 +3,8 @@
 //
 //   detect : the sphere path's half-stencil sweep (13 cells as 5 slot ranges)
 //            with the circumscribed-sphere test as single-precision
-//            pre-filter; each surviving pair runs the Johnson GJK distance
+//            pre-filter; a filter drops the pairs whose bodies are surely
+//            apart, and each remaining pair runs the Johnson GJK distance
 //            between the crust-shrunk bodies (RigidBodyWithCrust::ClosestPoint,
 //            Component/src/RigidBodyWithCrust.cpp:274-348) once, and the
 //            contact (point, overlap vector, overlap) is stored in the
@@ -53,33 +54,30 @@ __device__ __forceinline__ Orient load_orient(const CState& c, int s) {
 // (the first test of RigidBodyWithCrust::ClosestPoint) is queued; the GJK runs
 // in a second kernel with one lane per candidate, so lanes do not wait on
 // each other's narrow phase.
+//
+// kSweepLanes lanes sweep one particle together (eight for few particles, two
+// for many): each takes every kSweepLanes-th slot of a range and the kept candidates are appended in slot
+// order (ballot over the particle's lanes), so the lists are those of a
+// serial sweep.  The sweep is a chain of loads and tests, about 100 slots per
+// particle: with one lane per particle it took 35 us at 3,000 particles as at
+// 40,000.
+template <int kSweepLanes>
 struct CCandidates {
   const CDetectArgs& a;
-  int t;
+  int t, sub, shift;  // lane of the particle, its first lane in the wave
   float4 mef;
-  bool have_me;
   v3 X;
   double circ;
   int32_t id;
   int ncand;
 
-  __device__ __forceinline__ CCandidates(const CDetectArgs& a_, int t_, float4 mef_)
-      : a(a_), t(t_), mef(mef_), have_me(false), X{}, circ(0.), id(0), ncand(0) {}
-
-  __device__ __forceinline__ void test(const float4 p2f, int u, int sx, int sy, int sz, bool same) {
+  __device__ __forceinline__ bool test(int u, int sx, int sy, int sz, bool same, int& code) {
+    const float4 p2f = a.pos[u];
     const float dxf = (p2f.x + sx * a.sizef[0]) - mef.x;
     const float dyf = (p2f.y + sy * a.sizef[1]) - mef.y;
     const float dzf = (p2f.z + sz * a.sizef[2]) - mef.z;
     const float rsf = mef.w + p2f.w + a.margin;
-    if (dxf * dxf + dyf * dyf + dzf * dzf > rsf * rsf) return;
-    if (!have_me) {
-      const int s = a.perm[t];
-      const double4 p = a.in.pos_r[s];
-      X = mk(p.x, p.y, p.z);
-      circ = p.w;
-      id = a.in.aux[s].id;
-      have_me = true;
-    }
+    if (dxf * dxf + dyf * dyf + dzf * dzf > rsf * rsf) return false;
     const int s2 = a.perm[u];
     const double4 p2 = a.in.pos_r[s2];
     const int32_t id2 = a.in.aux[s2].id;
@@ -89,34 +87,52 @@ struct CCandidates {
     v3 gab;
     double cA, cB;
     if (first) {
-      gab = sub(X, mk(p2.x + shx, p2.y + shy, p2.z + shz));
+      gab = sub3(X, mk(p2.x + shx, p2.y + shy, p2.z + shz));
       cA = circ; cB = p2.w;
     } else {
-      gab = sub(mk(p2.x, p2.y, p2.z), mk(X.x + (-shx), X.y + (-shy), X.z + (-shz)));
+      gab = sub3(mk(p2.x, p2.y, p2.z), mk(X.x + (-shx), X.y + (-shy), X.z + (-shz)));
       cA = p2.w; cB = circ;
     }
-    if (!(norm(gab) < cA + cB)) return;
-    if (ncand >= kCandCap) {
-      atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)id);
-      return;
-    }
-    a.cand[(size_t)t * kCandCap + ncand] = make_int2(u, pack_code(sx, sy, sz, first));
-    ++ncand;
+    code = pack_code(sx, sy, sz, first);
+    return norm(gab) < cA + cB;
   }
+  // gdem::sub under a name the member does not hide
+  __device__ __forceinline__ v3 sub3(v3 p, v3 q) const { return gdem::sub(p, q); }
 
+  // The ranges differ between the particles of a wave: the lanes of one
+  // particle go through its own together.
   __device__ __forceinline__ void range(int beg, int end, int sx, int sy, int sz, bool same) {
-    for (int u = beg; u < end; ++u) test(a.pos[u], u, sx, sy, sz, same);
+    for (int u0 = beg; u0 < end; u0 += kSweepLanes) {
+      const int u = u0 + sub;
+      int code = 0;
+      const bool keep = u < end && test(u, sx, sy, sz, same, code);
+      const uint32_t who =
+          (uint32_t)(__ballot(keep) >> shift) & ((1u << kSweepLanes) - 1u);
+      const int at = ncand + __builtin_popcount(who & ((1u << sub) - 1u));
+      if (keep) {
+        if (at < kCandCap) a.cand[(size_t)t * kCandCap + at] = make_int2(u, code);
+        else atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)id);
+      }
+      ncand = min(ncand + __builtin_popcount(who), kCandCap);
+    }
   }
 };
 
-__global__ void __launch_bounds__(kCBlock) k_cdetect(CDetectArgs a) {
-  const int t = logical_index(a.nblk8);
+template <int kSweepLanes>
+__global__ void __launch_bounds__(kCBlock) k_cdetect(CDetectArgs a, int nblk8) {
+  __shared__ int sh_wave[kCBlock / 64], sh_base;
+  constexpr int P = kCBlock / kSweepLanes;  // particles per workgroup
+  const int lane = threadIdx.x & 63, sub = threadIdx.x % kSweepLanes;
+  const int t = ((blockIdx.x & 7) * (nblk8 >> 3) + (blockIdx.x >> 3)) * P +
+                threadIdx.x / kSweepLanes;
   int nc = 0;
   if (t < a.n) {
-    const double4 me = a.in.pos_r[a.perm[t]];
+    const int s = a.perm[t];
+    const double4 me = a.in.pos_r[s];
     int ijk[3];
     clamped_cell(a.grid, mk(me.x, me.y, me.z), ijk);
-    CCandidates det(a, t, a.pos[t]);
+    CCandidates<kSweepLanes> det{a,    t,    sub, lane - sub, a.pos[t], mk(me.x, me.y, me.z),
+                    me.w, a.in.aux[s].id, 0};
     half_stencil_sweep(a.grid, a.row_rank, a.cell_start, t, ijk, det);
     nc = det.ncand;
     // SimpleObstacle::InterAction's InZone test (Component/src/SimpleObstacle.cpp:222-271)
@@ -127,28 +143,121 @@ __global__ void __launch_bounds__(kCBlock) k_cdetect(CDetectArgs a) {
             fabs(wl.bb_centre[2] - me.z) <= wl.bb_ext[2] + me.w))
         continue;
       if (nc >= kCandCap) {
-        atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)a.in.aux[a.perm[t]].id);
+        atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)det.id);
         break;
       }
-      a.cand[(size_t)t * kCandCap + nc] = make_int2(wi, kWallCode);
+      if (sub == 0) a.cand[(size_t)t * kCandCap + nc] = make_int2(wi, kWallCode);
       ++nc;
     }
-    a.cand_count[t] = nc;
-    a.mask[t] = 0u;
+    if (sub == 0) {
+      a.cand_count[t] = nc;
+      a.mask[t] = 0u;
+    }
   }
-  // queue the candidates: one atomic per wave
-  const int lane = threadIdx.x & 63;
-  int incl = nc;
+  // queue the candidates: one atomic per workgroup
+  const int mine = sub == 0 ? nc : 0, wid = threadIdx.x >> 6;
+  int incl = mine;
   for (int o = 1; o < 64; o <<= 1) {
     const int y = __shfl_up(incl, o, 64);
     if (lane >= o) incl += y;
   }
-  const int total = __shfl(incl, 63, 64);
-  int base = 0;
-  if (lane == 63 && total > 0) base = atomicAdd(a.nwork, total);
-  base = __shfl(base, 63, 64);
-  const int off = base + incl - nc;
-  for (int j = 0; j < nc; ++j) a.work[off + j] = t * kCandCap + j;
+  if (lane == 63) sh_wave[wid] = incl;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int tot = 0;
+    for (int w = 0; w < kCBlock / 64; ++w) tot += sh_wave[w];
+    sh_base = tot ? atomicAdd(a.nwork, tot) : 0;
+  }
+  __syncthreads();
+  // the lanes of a particle share its part of the queue
+  int off = sh_base + __shfl(incl - mine, lane - sub, 64);
+  for (int w = 0; w < wid; ++w) off += sh_wave[w];
+  for (int j = sub; j < nc; j += kSweepLanes) a.work[off + j] = t * kCandCap + j;
+}
+
+// Support value of a shape (its crust-shrunk transform's linear part b) along
+// d, max over the body of d . (b p), and the support point b p itself.
+__device__ __forceinline__ v3 shrunk_support(const CShape& sh, const double* b, const double* sc,
+                                             v3 d) {
+  const v3 l = mk((b[0] * d.x + b[3] * d.y + b[6] * d.z) * sc[0],
+                  (b[1] * d.x + b[4] * d.y + b[7] * d.z) * sc[1],
+                  (b[2] * d.x + b[5] * d.y + b[8] * d.z) * sc[2]);
+  v3 p;
+  if (sh.type == SHAPE_BOX) {
+    p = mk(l.x < 0. ? -sh.ext[0] : sh.ext[0], l.y < 0. ? -sh.ext[1] : sh.ext[1],
+           l.z < 0. ? -sh.ext[2] : sh.ext[2]);
+  } else {
+    p = mk(sh.v[0][0], sh.v[0][1], sh.v[0][2]);
+    double h = dot(p, l);
+    for (int k = 1; k < sh.nv; ++k) {
+      const v3 q = mk(sh.v[k][0], sh.v[k][1], sh.v[k][2]);
+      const double hq = dot(q, l);
+      if (hq > h) {
+        h = hq;
+        p = q;
+      }
+    }
+  }
+  p = mk(p.x * sc[0], p.y * sc[1], p.z * sc[2]);
+  return mk(b[0] * p.x + b[1] * p.y + b[2] * p.z, b[3] * p.x + b[4] * p.y + b[5] * p.z,
+            b[6] * p.x + b[7] * p.y + b[8] * p.z);
+}
+
+// True when the crust-shrunk bodies are surely further apart than the crusts
+// together, so that the closest-point run would find no contact: a few
+// Frank-Wolfe steps towards the point v of their Minkowski difference nearest
+// the origin.  Each support point w bounds the distance from below by
+// v . w / |v|; the margin (a billionth of the bodies' size) dwarfs the
+// rounding of that bound and of the GJK's distance, which is the length of a
+// point of the difference and so never below the true distance by more.
+// False decides nothing.  d: centre of A minus centre of B (A at B's image).
+constexpr int kApartSteps = 6;
+__device__ __forceinline__ bool surely_apart(const CShape& shA, const double* bA,
+                                             const double* scA, const CShape& shB,
+                                             const double* bB, const double* scB, v3 d,
+                                             double reach) {
+  v3 v = d;
+  for (int k = 0; k < kApartSteps; ++k) {
+    const v3 w = add(d, sub(shrunk_support(shA, bA, scA, neg(v)), shrunk_support(shB, bB, scB, v)));
+    const double vw = dot(v, w), vv = dot(v, v);
+    if (vw > 0. && vw * vw > vv * (reach * reach)) return true;
+    if (vv <= reach * reach) return false;
+    const v3 e = sub(v, w);
+    const double ee = dot(e, e), step = dot(v, e);
+    if (!(step > 0.) || !(ee > 0.)) return false;
+    v = sub(v, scl(e, step < ee ? step / ee : 1.));
+  }
+  return false;
+}
+
+// The candidate surely has no contact (see surely_apart); rectangles are left
+// to their closed form.
+__device__ __forceinline__ bool candidate_apart(const CGjkArgs& a, int item) {
+  const int t = item / kCandCap;
+  const int2 cd = a.cand[item];
+  const int u = cd.x, code = cd.y;
+  const int s1 = a.perm[t];
+  const double4 p1 = a.in.pos_r[s1];
+  const Aux ax1 = a.in.aux[s1];
+  const Orient o1 = load_orient(a.cin, s1);
+  if (code == kWallCode) {
+    const Wall& wl = a.walls[u];
+    if (wl.kind == WALL_RECTANGLE) return false;
+    const double4 wsc = a.wall_sc[u];
+    const double wscale[3] = {wsc.x, wsc.y, wsc.z};
+    const v3 d = mk(p1.x - wl.origin[0], p1.y - wl.origin[1], p1.z - wl.origin[2]);
+    return surely_apart(a.shapes[aux_shape(ax1)], o1.b, o1.sc, a.wall_shapes[u], wl.basis, wscale,
+                        d, (ax1.crust + wl.crust) + 1e-9 * (p1.w + wsc.w));
+  }
+  const int sx = (code & 3) - 1, sy = ((code >> 2) & 3) - 1, sz = ((code >> 4) & 3) - 1;
+  const int s2 = a.perm[u];
+  const double4 p2 = a.in.pos_r[s2];
+  const Aux ax2 = a.in.aux[s2];
+  const Orient o2 = load_orient(a.cin, s2);
+  const v3 d = mk(p1.x - (p2.x + sx * a.grid.size[0]), p1.y - (p2.y + sy * a.grid.size[1]),
+                  p1.z - (p2.z + sz * a.grid.size[2]));
+  return surely_apart(a.shapes[aux_shape(ax1)], o1.b, o1.sc, a.shapes[aux_shape(ax2)], o2.b, o2.sc,
+                      d, (ax1.crust + ax2.crust) + 1e-9 * (p1.w + p2.w));
 }
 
 // Narrow phase of one candidate: RigidBodyWithCrust::ClosestPoint
@@ -157,74 +266,31 @@ __global__ void __launch_bounds__(kCBlock) k_cdetect(CDetectArgs a) {
 // SV: the signed-volume GJK (CollisionDetection Type="GJK_SV") instead of
 // the Johnson one.
 template <bool SV>
-__global__ void __launch_bounds__(kCBlock) k_cgjk(CGjkArgs a) {
-  const int nw = *a.nwork;
-  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < nw; k += gridDim.x * blockDim.x) {
-    const int item = a.work[k];
-    const int t = item / kCandCap, j = item - t * kCandCap;
-    const int2 cd = a.cand[item];
-    const int u = cd.x, code = cd.y;
-    if (code == kWallCode) {
-      // the particle is the first body, the wall box the second
-      const int s1 = a.perm[t];
-      const double4 p1 = a.in.pos_r[s1];
-      const Aux ax1 = a.in.aux[s1];
-      const Orient o1 = load_orient(a.cin, s1);
-      const Wall& wl = a.walls[u];
-      const double4 wsc = a.wall_sc[u];
-      const double wscale[3] = {wsc.x, wsc.y, wsc.z};
-      const CBody A{&a.shapes[aux_shape(ax1)], o1.b, mk(p1.x, p1.y, p1.z), o1.sc, ax1.crust, p1.w};
-      const CBody B{&a.wall_shapes[u], wl.basis, mk(wl.origin[0], wl.origin[1], wl.origin[2]),
-                    wscale, wl.crust, wsc.w};
-      v3 c = mk(0., 0., 0.), ov = mk(0., 0., 0.);
-      double dist = 0.;
-      int nit = 0;  // ClosestPointRECTANGLE reports none
-      int rc = wl.kind == WALL_RECTANGLE ? convex_rect(A, wl, c, ov, dist)
-                                         : closest_point<SV>(A, B, c, ov, dist, nit);
-      if (rc < 0) rc = closest_point_retry(A, B, c, ov, dist, nit);
-      if (rc < 0) {
-        atomicMin(&a.err[kErrContact], pack_ids(ax1.id, -1 - u));
-        continue;
-      }
-      if (a.stats) {
-        CRec& r = a.rec[item];
-        r.dist = dist;
-        r.nit = nit;
-        r.evaluated = rc != 0;
-      }
-      if (rc == 0 || !(dist < 0.)) continue;
-      CRec& r = a.rec[item];
-      r.c[0] = c.x; r.c[1] = c.y; r.c[2] = c.z;
-      r.ov[0] = ov.x; r.ov[1] = ov.y; r.ov[2] = ov.z;
-      r.dist = dist;
-      atomicOr(&a.mask[t], 1u << j);
-      continue;
-    }
-    const int sx = (code & 3) - 1, sy = ((code >> 2) & 3) - 1, sz = ((code >> 4) & 3) - 1;
-    const bool first = (code & 64) != 0;
-    const double shx = sx * a.grid.size[0], shy = sy * a.grid.size[1], shz = sz * a.grid.size[2];
-    const int s1 = a.perm[t], s2 = a.perm[u];
-    const double4 p1 = a.in.pos_r[s1], p2 = a.in.pos_r[s2];
-    const Aux ax1 = a.in.aux[s1], ax2 = a.in.aux[s2];
-    const Orient o1 = load_orient(a.cin, s1), o2 = load_orient(a.cin, s2);
-    CBody A, B;
-    if (first) {
-      A = CBody{&a.shapes[aux_shape(ax1)], o1.b, mk(p1.x, p1.y, p1.z), o1.sc, ax1.crust, p1.w};
-      B = CBody{&a.shapes[aux_shape(ax2)], o2.b, mk(p2.x + shx, p2.y + shy, p2.z + shz), o2.sc,
-                ax2.crust, p2.w};
-    } else {
-      A = CBody{&a.shapes[aux_shape(ax2)], o2.b, mk(p2.x, p2.y, p2.z), o2.sc, ax2.crust, p2.w};
-      B = CBody{&a.shapes[aux_shape(ax1)], o1.b, mk(p1.x + (-shx), p1.y + (-shy), p1.z + (-shz)),
-                o1.sc, ax1.crust, p1.w};
-    }
-    v3 c, ov;
+__device__ __forceinline__ void narrow_phase(const CGjkArgs& a, int item) {
+  const int t = item / kCandCap, j = item - t * kCandCap;
+  const int2 cd = a.cand[item];
+  const int u = cd.x, code = cd.y;
+  if (code == kWallCode) {
+    // the particle is the first body, the wall box the second
+    const int s1 = a.perm[t];
+    const double4 p1 = a.in.pos_r[s1];
+    const Aux ax1 = a.in.aux[s1];
+    const Orient o1 = load_orient(a.cin, s1);
+    const Wall& wl = a.walls[u];
+    const double4 wsc = a.wall_sc[u];
+    const double wscale[3] = {wsc.x, wsc.y, wsc.z};
+    const CBody A{&a.shapes[aux_shape(ax1)], o1.b, mk(p1.x, p1.y, p1.z), o1.sc, ax1.crust, p1.w};
+    const CBody B{&a.wall_shapes[u], wl.basis, mk(wl.origin[0], wl.origin[1], wl.origin[2]),
+                  wscale, wl.crust, wsc.w};
+    v3 c = mk(0., 0., 0.), ov = mk(0., 0., 0.);
     double dist = 0.;
-    int nit = 0;
-    int rc = closest_point<SV>(A, B, c, ov, dist, nit);
+    int nit = 0;  // ClosestPointRECTANGLE reports none
+    int rc = wl.kind == WALL_RECTANGLE ? convex_rect(A, wl, c, ov, dist)
+                                       : closest_point<SV>(A, B, c, ov, dist, nit);
     if (rc < 0) rc = closest_point_retry(A, B, c, ov, dist, nit);
     if (rc < 0) {
-      atomicMin(&a.err[kErrContact], first ? pack_ids(ax1.id, ax2.id) : pack_ids(ax2.id, ax1.id));
-      continue;
+      atomicMin(&a.err[kErrContact], pack_ids(ax1.id, -1 - u));
+      return;
     }
     if (a.stats) {
       CRec& r = a.rec[item];
@@ -232,19 +298,105 @@ __global__ void __launch_bounds__(kCBlock) k_cgjk(CGjkArgs a) {
       r.nit = nit;
       r.evaluated = rc != 0;
     }
-    if (rc == 0 || !(dist < 0.)) continue;
+    if (rc == 0 || !(dist < 0.)) return;
     CRec& r = a.rec[item];
     r.c[0] = c.x; r.c[1] = c.y; r.c[2] = c.z;
     r.ov[0] = ov.x; r.ov[1] = ov.y; r.ov[2] = ov.z;
     r.dist = dist;
     atomicOr(&a.mask[t], 1u << j);
-    const int kin = atomicAdd(&a.in_count[u], 1);
-    if (kin < kCandCap) {
-      a.in_list[(size_t)u * kCandCap + kin] = make_int2(t, j);
-    } else {
-      atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)ax2.id);
-    }
+    return;
   }
+  const int sx = (code & 3) - 1, sy = ((code >> 2) & 3) - 1, sz = ((code >> 4) & 3) - 1;
+  const bool first = (code & 64) != 0;
+  const double shx = sx * a.grid.size[0], shy = sy * a.grid.size[1], shz = sz * a.grid.size[2];
+  const int s1 = a.perm[t], s2 = a.perm[u];
+  const double4 p1 = a.in.pos_r[s1], p2 = a.in.pos_r[s2];
+  const Aux ax1 = a.in.aux[s1], ax2 = a.in.aux[s2];
+  const Orient o1 = load_orient(a.cin, s1), o2 = load_orient(a.cin, s2);
+  CBody A, B;
+  if (first) {
+    A = CBody{&a.shapes[aux_shape(ax1)], o1.b, mk(p1.x, p1.y, p1.z), o1.sc, ax1.crust, p1.w};
+    B = CBody{&a.shapes[aux_shape(ax2)], o2.b, mk(p2.x + shx, p2.y + shy, p2.z + shz), o2.sc,
+              ax2.crust, p2.w};
+  } else {
+    A = CBody{&a.shapes[aux_shape(ax2)], o2.b, mk(p2.x, p2.y, p2.z), o2.sc, ax2.crust, p2.w};
+    B = CBody{&a.shapes[aux_shape(ax1)], o1.b, mk(p1.x + (-shx), p1.y + (-shy), p1.z + (-shz)),
+              o1.sc, ax1.crust, p1.w};
+  }
+  v3 c, ov;
+  double dist = 0.;
+  int nit = 0;
+  int rc = closest_point<SV>(A, B, c, ov, dist, nit);
+  if (rc < 0) rc = closest_point_retry(A, B, c, ov, dist, nit);
+  if (rc < 0) {
+    atomicMin(&a.err[kErrContact], first ? pack_ids(ax1.id, ax2.id) : pack_ids(ax2.id, ax1.id));
+    return;
+  }
+  if (a.stats) {
+    CRec& r = a.rec[item];
+    r.dist = dist;
+    r.nit = nit;
+    r.evaluated = rc != 0;
+  }
+  if (rc == 0 || !(dist < 0.)) return;
+  CRec& r = a.rec[item];
+  r.c[0] = c.x; r.c[1] = c.y; r.c[2] = c.z;
+  r.ov[0] = ov.x; r.ov[1] = ov.y; r.ov[2] = ov.z;
+  r.dist = dist;
+  atomicOr(&a.mask[t], 1u << j);
+  const int kin = atomicAdd(&a.in_count[u], 1);
+  if (kin < kCandCap) {
+    a.in_list[(size_t)u * kCandCap + kin] = make_int2(t, j);
+  } else {
+    atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)ax2.id);
+  }
+}
+
+// Queued candidates that are not surely apart (most are: their circumscribed
+// spheres overlap, the bodies do not) to the queue of the narrow phase; one
+// integer atomic per workgroup.  With statistics on every candidate is
+// evaluated: its GJK iterations count.  A queue of at most kFilterFrom
+// candidates is left as it is: its waves run side by side, and the filter's
+// 20 us would come on top of the slowest one.
+constexpr int kFilterFrom = 32768;
+__global__ void __launch_bounds__(kCBlock) k_cfilter(CGjkArgs a) {
+  __shared__ int sh_wave[kCBlock / 64], sh_base;
+  const int nw = *a.nwork;
+  if (nw <= kFilterFrom) return;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  for (int k0 = blockIdx.x * kCBlock; k0 < nw; k0 += gridDim.x * kCBlock) {
+    const int k = k0 + threadIdx.x;
+    const int item = k < nw ? a.work[k] : 0;
+    const bool keep = k < nw && (a.stats || !candidate_apart(a, item));
+    const unsigned long long who = __ballot(keep);
+    if (lane == 0) sh_wave[wid] = __popcll(who);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int tot = 0;
+      for (int w = 0; w < kCBlock / 64; ++w) tot += sh_wave[w];
+      sh_base = tot ? atomicAdd(a.nnear, tot) : 0;
+    }
+    __syncthreads();
+    int at = sh_base + __popcll(who & ((1ull << lane) - 1ull));
+    for (int w = 0; w < wid; ++w) at += sh_wave[w];
+    if (keep) a.near[at] = item;
+    __syncthreads();
+  }
+}
+
+// Workgroups of one wave: the GJK holds all registers of a SIMD and a wave is
+// as slow as its slowest lane, so waves are spread over the compute units one
+// by one.  40,000 bodies at solid fraction 0.20 (160,000 candidates): 169 us
+// per launch over the whole queue in workgroups of four waves; filter 23 us
+// and 108 us for what it leaves.
+constexpr int kGjkBlock = 64;
+template <bool SV>
+__global__ void __launch_bounds__(kGjkBlock) k_cgjk(CGjkArgs a) {
+  const bool all = *a.nwork <= kFilterFrom;
+  const int nw = all ? *a.nwork : *a.nnear;
+  const int32_t* queue = all ? a.work : a.near;
+  for (int k = blockIdx.x * kGjkBlock + threadIdx.x; k < nw; k += gridDim.x * kGjkBlock)
+    narrow_phase<SV>(a, queue[k]);
 }
 
 // ---------------------------------------------------------------- force
@@ -398,7 +550,7 @@ __global__ void __launch_bounds__(kCBlock) k_cforce(CForceArgs a) {
     R.T = mk(0., 0., 0.);
     R.ncont = 0;
     R.nrec = 0;
-    if (t == 0) *a.nwork = 0;  // the candidate queue of the next step starts empty
+    if (t == 0) a.nwork[0] = a.nwork[1] = 0;  // the candidate queue of the next step starts empty
     // own contacts in sweep order, then the received ones by increasing
     // (detecting slot, candidate index)
     uint32_t mk_bits = a.mask[t];
@@ -582,17 +734,23 @@ static inline int cblocks(int n) { return (n + kCBlock - 1) / kCBlock; }
 
 void launch_cdetect(const CDetectArgs& a, hipStream_t st) {
   if (a.n <= 0) return;
-  hipLaunchKernelGGL(k_cdetect, dim3(a.nblk8), dim3(kCBlock), 0, st, a);
+  const bool few = a.n < 32768;
+  const int p = kCBlock / (few ? 8 : 2);
+  const int nblk8 = ((a.n + p - 1) / p + 7) / 8 * 8;
+  if (few) hipLaunchKernelGGL(k_cdetect<8>, dim3(nblk8), dim3(kCBlock), 0, st, a, nblk8);
+  else hipLaunchKernelGGL(k_cdetect<2>, dim3(nblk8), dim3(kCBlock), 0, st, a, nblk8);
 }
 
 void launch_cgjk(const CGjkArgs& a, int32_t max_work, hipStream_t st) {
   if (max_work <= 0) return;
-  // grid-stride over the queue; the grid covers a typical queue in one pass
-  const int blocks = std::min(std::max(cblocks(max_work), 1), 16384);
+  // grid-stride over the queues; the grids cover typical ones in one pass
+  hipLaunchKernelGGL(k_cfilter, dim3(std::min(std::max(cblocks(max_work), 1), 16384)),
+                     dim3(kCBlock), 0, st, a);
+  const int waves = std::min(std::max(max_work / kGjkBlock, 1), 16384);
   if (a.gjk_sv)
-    hipLaunchKernelGGL(k_cgjk<true>, dim3(blocks), dim3(kCBlock), 0, st, a);
+    hipLaunchKernelGGL(k_cgjk<true>, dim3(waves), dim3(kGjkBlock), 0, st, a);
   else
-    hipLaunchKernelGGL(k_cgjk<false>, dim3(blocks), dim3(kCBlock), 0, st, a);
+    hipLaunchKernelGGL(k_cgjk<false>, dim3(waves), dim3(kGjkBlock), 0, st, a);
 }
 
 void launch_cforce(int mode, bool record, const CForceArgs& a, hipStream_t st) {

@@ -317,6 +317,8 @@ struct CGjkArgs {
   const int2* cand;
   const int32_t* work;
   const int32_t* nwork;
+  int32_t* near;       // candidates not surely apart: the narrow phase's queue
+  int32_t* nnear;      // its length (zero on entry)
   const Wall* walls;
   const CShape* wall_shapes;  // box shape of each wall
   const double4* wall_sc;     // crust scaling per axis, circumscribed radius
@@ -347,7 +349,7 @@ struct CForceArgs {
   const uint32_t* mask;
   const int2* in_list;
   int32_t* in_count;
-  int32_t* nwork;      // reset to zero for the next step
+  int32_t* nwork;      // both queue lengths, reset to zero for the next step
   StatPart* stat;      // contact statistics, one part per workgroup (nullable)
   double4* F;
   double4* T;
