@@ -48,6 +48,11 @@ struct DiffSys {
   double gravity[3];
   int32_t n, off, cell_off, cs_off, row_off, wall_off, nwalls;
   int32_t substeps;  // steps of dt / substeps per step of dt
+  double skin;       // candidate lists hold every pair with a gap below it; 0:
+                     // contact lists, rebuilt at every evaluation
+  double limit2;     // (skin / 2)^2, less a relative 2e-6
+  Grid lgrid;        // cells of the candidate lists: two radii and the skin
+  int32_t lrow_off;
   double kn, en, mu, beta, dbeta;  // beta(en) and d beta / d en
 };
 
@@ -64,6 +69,12 @@ struct DiffArgs {
   int64_t ntot;
   const double4* prop;  // r, m, I, crust
   Aux* aux;
+  double4* xref;        // positions the candidate lists were built from
+  // contacts of the current evaluation, by particle in the order of summation:
+  // [2 kListCap][n] per system (partner, code), their ranks, their number
+  int2* con;
+  long long* con_rank;
+  int32_t* con_count;
   const double4* x0;    // initial x, y, z, r
   const double4* v0;
   const double4* w0;
@@ -174,6 +185,7 @@ struct DiffRunner {
   // a stiff system advances sub steps of dt / sub per step: nst steps of dt
   // in all, checkpoints every Ks of them, observation k after obs[k] * sub
   int sub = 1, nst = 0, Ks = 0;
+  double skin = 0.;  // sy.skin; 0 once a candidate list overflowed
   double dt = 0.;
 
   __device__ __forceinline__ unsigned long long* err() const { return a.err + (size_t)s * kErrWords; }
@@ -198,98 +210,224 @@ struct DiffRunner {
   __device__ __forceinline__ double4* To() const { return a.T + sy.off; }
   __device__ __forceinline__ const double4* P() const { return a.prop + sy.off; }
 
-  // Keys of the current positions, counting sort by cell (ties by id), sorted
-  // float copy, half-stencil detection: contact lists by slot.
-  __device__ __forceinline__ void bin_and_detect() {
-    const int n = sy.n, nc = sy.grid.ncell;
-    int32_t* key = a.key + sy.off;
-    int32_t* slot = a.slot + sy.off;
-    int32_t* perm = a.perm + sy.off;
-    int32_t* cnt = a.cnt + sy.cell_off;
-    int32_t* cs = a.cell_start + sy.cs_off;
-    const int32_t* rr = a.row_rank + sy.row_off;
+  // Contact lists of the current positions, from candidate lists (Verlet
+  // lists) kept while no particle is further than skin / 2 from where they
+  // were built, so every pair that may touch is listed.  Candidates that
+  // overflow a list hold the contacts alone from then on, as they do where the
+  // cells leave no room for a skin.  Binning and sweeping at every evaluation
+  // took half of a gradient, serial phases of few memory accesses each: 512
+  // systems of 1,000 over 400 steps 672 ms with them, 494 ms so; 12 of 250
+  // over 60 steps 21.7 and 13.9 ms.  first: the first evaluation of a launch.
+  __device__ __forceinline__ void lists(bool first = false) {
+    const int n = sy.n;
+    if (threadIdx.x == 0) smem[1] = first || !(skin > 0.) ? 1 : 0;
+    __syncthreads();
     for (int i = threadIdx.x; i < n; i += BS) {
       const double4 p = X()[i];
       int ijk[3];
-      if (!cell_of(sy.grid, mk(p.x, p.y, p.z), ijk)) {
+      if (!cell_of(sy.grid, mk(p.x, p.y, p.z), ijk))
         atomicMin(&err()[kErrSim], (unsigned long long)(uint32_t)i);
-        key[i] = 0;
-      } else {
-        key[i] = row_base(sy.grid, rr, ijk[1], ijk[2]) + ijk[0];
+      if (!first) {
+        const double4 q = a.xref[sy.off + i];
+        const double dx = p.x - q.x, dy = p.y - q.y, dz = p.z - q.z;
+        if (!(dx * dx + dy * dy + dz * dz <= sy.limit2)) smem[1] = 1;
       }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < n; i += BS) slot[i] = atomicAdd(&cnt[key[i]], 1);
+    const bool due = smem[1] != 0;
     __syncthreads();
-    int carry = 0;
-    for (int base = 0; base < nc; base += BS) {
-      const int c = base + threadIdx.x;
-      const int v = c < nc ? cnt[c] : 0;
-      int total;
-      const int ex = block_scan_excl_d<BS>(v, smem, total);
-      if (c < nc) {
-        cs[c] = carry + ex;
-        cnt[c] = 0;
-      }
-      carry += total;
-    }
-    if (threadIdx.x == 0) cs[nc] = n;
-    __syncthreads();
-    for (int i = threadIdx.x; i < n; i += BS) perm[cs[key[i]] + slot[i]] = i;
-    __syncthreads();
-    for (int c = threadIdx.x; c < nc; c += BS) {
-      const int beg = cs[c], end = cs[c + 1];
-      for (int q = beg + 1; q < end; ++q) {
-        const int v = perm[q];
-        int b = q - 1;
-        while (b >= beg && perm[b] > v) {
-          perm[b + 1] = perm[b];
-          --b;
+    if (due) build_lists();
+    contacts();
+  }
+
+  // The candidates that may touch, each particle's own (pairs a sweep of the
+  // cells of the current positions finds from its cell) in the order of that
+  // sweep, then the others by (partner's cell key, id): the sums, and with
+  // them every result, do not depend on when the candidates were listed.
+  __device__ __forceinline__ void contacts() {
+    const int n = sy.n;
+    const int32_t* perm = a.perm + sy.off;
+    const int32_t* rr = a.row_rank + sy.row_off;
+    for (int t = threadIdx.x; t < n; t += BS) {
+      const int p = perm[t];
+      const double4 me = X()[p];
+      int2* con = a.con + (size_t)sy.off * 2 * kListCap + p;
+      long long* rank = a.con_rank + (size_t)sy.off * 2 * kListCap + p;
+      int ci[3];
+      bool have = false;
+      int nown = 0, nother = 0;
+      auto one = [&](int u, int code) {
+        const int q = perm[u];
+        const int s3[3] = {(code & 3) - 1, ((code >> 2) & 3) - 1, ((code >> 4) & 3) - 1};
+        const double4 o = X()[q];
+        const v3 sh = mk(s3[0] * sy.grid.size[0], s3[1] * sy.grid.size[1], s3[2] * sy.grid.size[2]);
+        const v3 O = mk(o.x + sh.x, o.y + sh.y, o.z + sh.z);
+        const double dx = O.x - me.x, dy = O.y - me.y, dz = O.z - me.z, rs = me.w + o.w;
+        if (dx * dx + dy * dy + dz * dz > rs * rs * (1. + 1e-10)) return;
+        if (!have) clamped_cell(sy.grid, mk(me.x, me.y, me.z), ci);
+        have = true;
+        int cq[3], dd[3];
+        clamped_cell(sy.grid, mk(o.x, o.y, o.z), cq);
+        bool nb = true;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          dd[k] = cq[k] + s3[k] * sy.grid.nc[k] - ci[k];
+          nb &= dd[k] >= -1 && dd[k] <= 1;
         }
-        perm[b + 1] = v;
-      }
+        if (!nb) return;
+        // rows of the half stencil in sweep order: (0, 0), (0, 1), (1, -1), (1, 0), (1, 1)
+        const int row = 3 * dd[1] + dd[2];
+        const bool own = row > 0 || (row == 0 && (dd[0] > 0 || (dd[0] == 0 && p < q)));
+        long long rk;
+        if (own) {
+          v3 c, ov;
+          double dist;
+          const double crA = P()[p].w, crB = P()[q].w;
+          int it, rc = sphere_sphere(mk(me.x, me.y, me.z), me.w, crA, O, o.w, crB, c, ov, dist);
+          if (rc < 0)
+            rc = sphere_sphere_retry(mk(me.x, me.y, me.z), me.w, crA, O, o.w, crB, c, ov, dist, it);
+          if (rc < 0) atomicMin(&err()[kErrContact], pack_ids(p, q));
+          if (rc <= 0 || !(dist < 0.)) return;
+          if (nown == kListCap) {
+            atomicMin(&err()[kErrCapacity], (unsigned long long)(uint32_t)p);
+            return;
+          }
+          rk = ((long long)(3 * row + dd[0] + 1) << 32) | q;
+        } else {
+          if (nother == kListCap) {
+            atomicMin(&err()[kErrCapacity], (unsigned long long)(uint32_t)p);
+            return;
+          }
+          rk = (1ll << 62) | ((long long)(row_base(sy.grid, rr, cq[1], cq[2]) + cq[0]) << 32) | q;
+        }
+        int b = nown + nother;
+        for (; b > 0 && rank[(size_t)(b - 1) * n] > rk; --b) {
+          rank[(size_t)b * n] = rank[(size_t)(b - 1) * n];
+          con[(size_t)b * n] = con[(size_t)(b - 1) * n];
+        }
+        rank[(size_t)b * n] = rk;
+        con[(size_t)b * n] = make_int2(q, pack_code(s3[0], s3[1], s3[2], own));
+        own ? ++nown : ++nother;
+      };
+      const int nout = min(a.out_count[sy.off + t], kListCap);
+      const int2* ol = a.out_list + (size_t)sy.off * kListCap + t;
+      for (int e = 0; e < nout; ++e) one(ol[(size_t)e * n].x, ol[(size_t)e * n].y);
+      const int nin = min(a.in_count[sy.off + t], kListCap);
+      const int2* il = a.in_list + (size_t)sy.off * kListCap + t;
+      for (int e = 0; e < nin; ++e) one(il[(size_t)e * n].x, il[(size_t)e * n].y);
+      a.con_count[sy.off + p] = nown + nother;
     }
-    __syncthreads();
-    float4* pos = a.pos + sy.off;
-    for (int u = threadIdx.x; u < n; u += BS) {
-      const double4 p = X()[perm[u]];
-      pos[u] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
-    }
-    if (threadIdx.x == 0) {
-      DetectArgs& d = *sd;
-      d.pos = pos;
-      d.sizef[0] = sy.sizef[0]; d.sizef[1] = sy.sizef[1]; d.sizef[2] = sy.sizef[2];
-      d.margin = sy.margin;
-      d.in.pos_r = X();
-      d.in.aux = a.aux + sy.off;
-      d.perm = perm;
-      d.cell_start = cs;
-      d.row_rank = rr;
-      d.grid = sy.grid;
-      d.n = n;
-      d.lstride = n;
-      d.out_list = a.out_list + (size_t)sy.off * kListCap;
-      d.out_count = a.out_count + sy.off;
-      d.in_list = a.in_list + (size_t)sy.off * kListCap;
-      d.in_count = a.in_count + sy.off;
-      d.err = err();
-      d.nblk8 = 0;
-      d.skin = 0.;
-      d.gate = SkinGate{};
-    }
-    __syncthreads();
-    for (int t = threadIdx.x; t < n; t += BS) detect_particle(*sd, t);
     __syncthreads();
   }
 
-  // Body order and image of one list entry of particle p (slot t): returns
-  // the partner id; meA tells whether p is the first body; shift is added to
-  // the partner (if p is A) or to p (if p is B).
-  __device__ __forceinline__ int decode(int u, int code, bool& meA, v3& shift) const {
+  // Keys of the current positions, counting sort by cell (ties by id), sorted
+  // float copy, half-stencil sweep: lists by slot.
+  __device__ __forceinline__ void build_lists() {
+    int32_t* perm = a.perm + sy.off;
+    for (;;) {
+      const bool wide = skin > 0.;
+      const int n = sy.n;
+      const Grid& g = wide ? sy.lgrid : sy.grid;
+      const int nc = g.ncell;
+      int32_t* key = a.key + sy.off;
+      int32_t* slot = a.slot + sy.off;
+      int32_t* cnt = a.cnt + sy.cell_off;
+      int32_t* cs = a.cell_start + sy.cs_off;
+      const int32_t* rr = a.row_rank + (wide ? sy.lrow_off : sy.row_off);
+      for (int i = threadIdx.x; i < n; i += BS) {
+        const double4 p = X()[i];
+        int ijk[3];
+        const bool in = cell_of(g, mk(p.x, p.y, p.z), ijk);
+        key[i] = in ? row_base(g, rr, ijk[1], ijk[2]) + ijk[0] : 0;
+        a.xref[sy.off + i] = p;
+        a.in_count[sy.off + i] = 0;
+      }
+      __syncthreads();
+      for (int i = threadIdx.x; i < n; i += BS) slot[i] = atomicAdd(&cnt[key[i]], 1);
+      __syncthreads();
+      int carry = 0;
+      for (int base = 0; base < nc; base += BS) {
+        const int c = base + threadIdx.x;
+        const int v = c < nc ? cnt[c] : 0;
+        int total;
+        const int ex = block_scan_excl_d<BS>(v, smem, total);
+        if (c < nc) {
+          cs[c] = carry + ex;
+          cnt[c] = 0;
+        }
+        carry += total;
+      }
+      if (threadIdx.x == 0) cs[nc] = n;
+      __syncthreads();
+      for (int i = threadIdx.x; i < n; i += BS) perm[cs[key[i]] + slot[i]] = i;
+      __syncthreads();
+      for (int c = threadIdx.x; c < nc; c += BS) {
+        const int beg = cs[c], end = cs[c + 1];
+        for (int q = beg + 1; q < end; ++q) {
+          const int v = perm[q];
+          int b = q - 1;
+          while (b >= beg && perm[b] > v) {
+            perm[b + 1] = perm[b];
+            --b;
+          }
+          perm[b + 1] = v;
+        }
+      }
+      __syncthreads();
+      float4* pos = a.pos + sy.off;
+      for (int u = threadIdx.x; u < n; u += BS) {
+        const double4 p = X()[perm[u]];
+        pos[u] = make_float4((float)p.x, (float)p.y, (float)p.z, (float)p.w);
+      }
+      if (threadIdx.x == 0) {
+        DetectArgs& d = *sd;
+        d.pos = pos;
+        d.sizef[0] = sy.sizef[0]; d.sizef[1] = sy.sizef[1]; d.sizef[2] = sy.sizef[2];
+        d.margin = sy.margin;
+        d.in.pos_r = X();
+        d.in.aux = a.aux + sy.off;
+        d.perm = perm;
+        d.ids = perm;  // particles are in id order
+        d.cell_start = cs;
+        d.row_rank = rr;
+        d.grid = g;
+        d.n = n;
+        d.lstride = n;
+        d.out_list = a.out_list + (size_t)sy.off * kListCap;
+        d.out_count = a.out_count + sy.off;
+        d.in_list = a.in_list + (size_t)sy.off * kListCap;
+        d.in_count = a.in_count + sy.off;
+        d.err = err();
+        d.nblk8 = 0;
+        d.skin = skin;
+        d.gap_unit = 1.f;  // the entries' gap bounds are not used
+        d.gate = SkinGate{};
+        smem[1] = 0;
+      }
+      __syncthreads();
+      for (int t = threadIdx.x; t < n; t += BS) detect_particle(*sd, t);
+      __syncthreads();
+      if (!wide) break;
+      for (int t = threadIdx.x; t < n; t += BS)
+        if (a.out_count[sy.off + t] > kListCap || a.in_count[sy.off + t] > kListCap) smem[1] = 1;
+      __syncthreads();
+      if (smem[1] == 0) break;
+      // candidates that do not fit are no error, contacts are
+      skin = 0.;
+      if (threadIdx.x == 0)
+        __hip_atomic_store(&err()[kErrCapacity], kNoErr, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+    }
+    __syncthreads();
+  }
+
+  // Body order and image of one contact: meA tells whether the particle is
+  // the first body; shift is added to the partner (if it is) or to the particle.
+  __device__ __forceinline__ void decode(int code, bool& meA, v3& shift) const {
     const int sx = (code & 3) - 1, sy_ = ((code >> 2) & 3) - 1, sz = ((code >> 4) & 3) - 1;
     meA = (code & 64) != 0;
     shift = mk(sx * sy.grid.size[0], sy_ * sy.grid.size[1], sz * sy.grid.size[2]);
-    return a.perm[sy.off + u];
   }
 
   __device__ __forceinline__ PairIn pair_in(int p, int q, bool meA, v3 shift) const {
@@ -320,16 +458,15 @@ struct DiffRunner {
   __device__ __forceinline__ void forces() {
     const int n = sy.n;
     const HookeParams<double> hp = params();
-    for (int t = threadIdx.x; t < n; t += BS) {
-      const int p = a.perm[sy.off + t];
+    for (int p = threadIdx.x; p < n; p += BS) {
       const double4 pp = P()[p];
       const double mw = pp.y * (1. - 0. / 1.);
       v3 F = mk(sy.gravity[0] * mw, sy.gravity[1] * mw, sy.gravity[2] * mw);
       v3 T = mk(0., 0., 0.);
-      auto one = [&](int u, int code) {
+      auto one = [&](int q, int code) {
         bool meA;
         v3 shift;
-        const int q = decode(u, code, meA, shift);
+        decode(code, meA, shift);
         const PairIn in = pair_in(p, q, meA, shift);
         V3<double> FA, TA, FB, TB;
         if (!pair_torsors(lift3<double>(in.xA), lift3<double>(in.vA), lift3<double>(in.wA), in.rA,
@@ -344,20 +481,9 @@ struct DiffRunner {
           T = add(T, val3(TB));
         }
       };
-      const int nout = min(a.out_count[sy.off + t], kListCap);
-      const int2* ol = a.out_list + (size_t)sy.off * kListCap + t;
-      for (int e = 0; e < nout; ++e) one(ol[(size_t)e * sy.n].x, ol[(size_t)e * sy.n].y);
-      const int nin = min(a.in_count[sy.off + t], kListCap);
-      a.in_count[sy.off + t] = 0;
-      const int2* il = a.in_list + (size_t)sy.off * kListCap + t;
-      long long last = -1;
-      for (int e = 0; e < nin; ++e) {
-        long long k;
-        const int f = next_incoming(il, nin, sy.n, last, k);
-        if (f < 0) break;
-        one(il[(size_t)f * sy.n].x, il[(size_t)f * sy.n].y);
-        last = k;
-      }
+      const int nc = a.con_count[sy.off + p];
+      const int2* con = a.con + (size_t)sy.off * 2 * kListCap + p;
+      for (int e = 0; e < nc; ++e) one(con[(size_t)e * sy.n].x, con[(size_t)e * sy.n].y);
       const v3 x = ld3(X()[p]), vv = ld3(V()[p]), ww = ld3(W()[p]);
       for (int wi = 0; wi < sy.nwalls; ++wi) {
         const Wall& wl = a.walls[sy.wall_off + wi];
@@ -457,13 +583,12 @@ struct DiffRunner {
     const int n = sy.n;
     const v3 tp = dtheta_beta();
     const double4 *tx = a.ax + sy.off, *tv = a.av + sy.off, *tw = a.aw + sy.off;
-    for (int t = threadIdx.x; t < n; t += BS) {
-      const int p = a.perm[sy.off + t];
+    for (int p = threadIdx.x; p < n; p += BS) {
       v3 dF = mk(0., 0., 0.), dT = mk(0., 0., 0.);
-      auto one = [&](int u, int code) {
+      auto one = [&](int q, int code) {
         bool meA;
         v3 shift;
-        const int q = decode(u, code, meA, shift);
+        decode(code, meA, shift);
         const PairIn in = pair_in(p, q, meA, shift);
         const int A = meA ? p : q, B = meA ? q : p;
         PairTan tin;
@@ -475,12 +600,9 @@ struct DiffRunner {
           dT = add(dT, tq);
         }
       };
-      const int nout = min(a.out_count[sy.off + t], kListCap);
-      const int2* ol = a.out_list + (size_t)sy.off * kListCap + t;
-      for (int e = 0; e < nout; ++e) one(ol[(size_t)e * sy.n].x, ol[(size_t)e * sy.n].y);
-      const int nin = min(a.in_count[sy.off + t], kListCap);
-      const int2* il = a.in_list + (size_t)sy.off * kListCap + t;
-      for (int e = 0; e < nin; ++e) one(il[(size_t)e * sy.n].x, il[(size_t)e * sy.n].y);
+      const int nc = a.con_count[sy.off + p];
+      const int2* con = a.con + (size_t)sy.off * 2 * kListCap + p;
+      for (int e = 0; e < nc; ++e) one(con[(size_t)e * sy.n].x, con[(size_t)e * sy.n].y);
       const double4 pp = P()[p];
       const v3 x = ld3(X()[p]), vv = ld3(V()[p]), ww = ld3(W()[p]);
       const v3 dx = ld3(tx[p]), dvv = ld3(tv[p]), dww = ld3(tw[p]);
@@ -537,7 +659,7 @@ struct DiffRunner {
     constexpr bool tan = TAN;
     if (tan) tangent_kick_drift();
     kick_drift();
-    bin_and_detect();
+    lists();
     if (j >= 0) {
       for (int i = threadIdx.x; i < sy.n; i += BS) {
         a.win_x[(size_t)j * a.ntot + sy.off + i] = X()[i];
@@ -545,7 +667,7 @@ struct DiffRunner {
         a.win_w[(size_t)j * a.ntot + sy.off + i] = W()[i];
       }
     }
-    if (tan) tangent_forces();  // reads in_count before forces() clears it
+    if (tan) tangent_forces();
     forces();
     if (tan) tangent_kick();
     kick();
@@ -575,13 +697,12 @@ struct DiffRunner {
     const int n = sy.n;
     const double4* aFt = a.aFt + sy.off;
     const double4* aTt = a.aTt + sy.off;
-    for (int t = threadIdx.x; t < n; t += BS) {
-      const int p = a.perm[sy.off + t];
+    for (int p = threadIdx.x; p < n; p += BS) {
       v3 dx = mk(0., 0., 0.), dv = mk(0., 0., 0.), dw = mk(0., 0., 0.);
-      auto one = [&](int u, int code, bool own) {
+      auto one = [&](int q, int code) {
         bool meA;
         v3 shift;
-        const int q = decode(u, code, meA, shift);
+        decode(code, meA, shift);
         const PairIn in = pair_in(p, q, meA, shift);
         const int A = meA ? p : q, B = meA ? q : p;
         PairAdj adj;
@@ -594,22 +715,11 @@ struct DiffRunner {
         dx = add(dx, meA ? pg.xA : pg.xB);
         dv = add(dv, meA ? pg.vA : pg.vB);
         dw = add(dw, meA ? pg.wA : pg.wB);
-        if (own) gth = add(gth, pg.th);
+        if (meA) gth = add(gth, pg.th);
       };
-      const int nout = min(a.out_count[sy.off + t], kListCap);
-      const int2* ol = a.out_list + (size_t)sy.off * kListCap + t;
-      for (int e = 0; e < nout; ++e) one(ol[(size_t)e * sy.n].x, ol[(size_t)e * sy.n].y, true);
-      const int nin = min(a.in_count[sy.off + t], kListCap);
-      a.in_count[sy.off + t] = 0;
-      const int2* il = a.in_list + (size_t)sy.off * kListCap + t;
-      long long last = -1;
-      for (int e = 0; e < nin; ++e) {
-        long long k;
-        const int f = next_incoming(il, nin, sy.n, last, k);
-        if (f < 0) break;
-        one(il[(size_t)f * sy.n].x, il[(size_t)f * sy.n].y, false);
-        last = k;
-      }
+      const int nc = a.con_count[sy.off + p];
+      const int2* con = a.con + (size_t)sy.off * 2 * kListCap + p;
+      for (int e = 0; e < nc; ++e) one(con[(size_t)e * sy.n].x, con[(size_t)e * sy.n].y);
       const double4 pp = P()[p];
       const v3 x = ld3(X()[p]), vv = ld3(V()[p]), ww = ld3(W()[p]);
       const v3 aF = ld3(aFt[p]), aT = ld3(aTt[p]);
@@ -655,7 +765,7 @@ struct DiffRunner {
       a.aTt[sy.off + i] = st3(add(ld3(aT[i]), scl(ld3(aw[i]), hdt / pp.z)), 0.);
     }
     __syncthreads();
-    bin_and_detect();
+    lists();
     force_vjp(a.gX, a.gV, a.gW);
     // drift x' = x + v_h dt and first kick v_h = v + (F/m) dt/2, w_h = w + (T/I) dt/2
     for (int i = threadIdx.x; i < sy.n; i += BS) {
@@ -688,10 +798,11 @@ struct DiffRunner {
     sub = sy.substeps;
     dt = a.dt / (double)sub;
     nst = a.nsteps * sub;
+    skin = sy.skin;
     Ks = a.K * sub;
     const double lscale = 1. / ((double)a.nobs * 3. * (double)sy.n);
     initial_state();
-    bin_and_detect();
+    lists(true);
     if constexpr (TAN) {
       // tangents of the initial state: positions fixed, velocities along the
       // given direction (in gv0), angular velocities fixed
@@ -749,7 +860,7 @@ struct DiffRunner {
       a.aTt[sy.off + i] = a.aT[sy.off + i];
     }
     __syncthreads();
-    bin_and_detect();
+    lists(true);
     force_vjp(a.gX, a.gV, a.gW);
     for (int i = threadIdx.x; i < sy.n; i += BS)
       a.gv0[sy.off + i] = st3(add(ld3(a.av[sy.off + i]), ld3(a.gV[sy.off + i])), 0.);
@@ -814,6 +925,10 @@ struct gdem_diff {
   double4 *d_prop = nullptr, *d_x0 = nullptr, *d_v0 = nullptr, *d_w0 = nullptr;
   Aux* d_aux = nullptr;
   double4 *d_x = nullptr, *d_v = nullptr, *d_w = nullptr, *d_F = nullptr, *d_T = nullptr;
+  double4* d_xref = nullptr;
+  int2* d_con = nullptr;
+  long long* d_con_rank = nullptr;
+  int32_t* d_con_count = nullptr;
   double4 *d_ck = nullptr, *d_win = nullptr, *d_target = nullptr, *d_xobs = nullptr;
   int32_t *d_key = nullptr, *d_slot = nullptr, *d_perm = nullptr, *d_cnt = nullptr, *d_cs = nullptr,
           *d_rows = nullptr, *d_out_count = nullptr, *d_in_count = nullptr;
@@ -855,7 +970,7 @@ extern "C" int gdem_diff_destroy(gdem_diff* d) {
   if (d->stream) (void)hipStreamSynchronize(d->stream);
   // d_v, d_w, d_F, d_T point into the d_x allocation
   void* ptrs[] = {d->d_sys, d->d_order, d->d_next, d->d_obs, d->d_prop, d->d_x0, d->d_v0, d->d_w0,
-                  d->d_aux, d->d_x, d->d_ck, d->d_win, d->d_target,
+                  d->d_aux, d->d_x, d->d_xref, d->d_con, d->d_con_rank, d->d_con_count, d->d_ck, d->d_win, d->d_target,
                   d->d_xobs, d->d_key, d->d_slot, d->d_perm, d->d_cnt, d->d_cs, d->d_rows,
                   d->d_out_count, d->d_in_count, d->d_pos, d->d_out_list, d->d_in_list, d->d_walls,
                   d->d_adj, d->d_loss, d->d_gtheta, d->d_err};
@@ -872,6 +987,9 @@ static void beta_of(double en, double& beta, double& dbeta) {
   beta = L / sqrt(kPi * kPi + L * L);
   dbeta = kPi * kPi / (en * pow(kPi * kPi + L * L, 1.5));
 }
+
+// Skin of the candidate lists in units of the largest radius.
+constexpr double kDiffSkin = 0.2;
 
 extern "C" int gdem_diff_add_system(gdem_diff* d, const gdem_batch_system* in, int32_t* sys_id) {
   if (!d || !in || d->committed) return GDEM_ERR_ARG;
@@ -890,6 +1008,19 @@ extern "C" int gdem_diff_add_system(gdem_diff* d, const gdem_batch_system* in, i
   DiffSys sy{};
   sy.substeps = std::max<int32_t>(in->substeps, 1);
   if (!make_grid(in->cfg, sy.grid)) return GDEM_ERR_ARG;
+  // the lists take cells that hold two radii and the skin, where the domain
+  // allows them (three along a periodic direction)
+  double rmax = 0.;
+  for (int64_t i = 0; i < n; ++i)
+    if (in->radius[i] > rmax) rmax = in->radius[i];
+  gdem_config wide = in->cfg;
+  wide.cell_size = std::max(wide.cell_size, 2. * rmax * (1. + 1e-9) + kDiffSkin * rmax);
+  if (!make_grid(wide, sy.lgrid) || sy.lgrid.ncell > sy.grid.ncell) sy.lgrid = sy.grid;
+  double edge = sy.lgrid.edge[0];
+  for (int k = 1; k < 3; ++k) edge = std::min(edge, sy.lgrid.edge[k]);
+  sy.skin = std::min(kDiffSkin * rmax, edge - 2. * rmax * (1. + 1e-9));
+  sy.limit2 = 0.25 * sy.skin * sy.skin * (1. - 2e-6);
+  if (!(sy.skin >= 0.02 * rmax)) sy.skin = 0.;
   sy.margin = prefilter_margin(sy.grid, sy.sizef);
   for (int k = 0; k < 3; ++k) sy.gravity[k] = in->cfg.gravity[k];
   sy.n = (int32_t)n;
@@ -907,6 +1038,9 @@ extern "C" int gdem_diff_add_system(gdem_diff* d, const gdem_batch_system* in, i
     if (!(in->radius[i] > 0.) || !(in->density[i] > 0.) || !(in->crust[i] > 0.)) return GDEM_ERR_ARG;
   const std::vector<int32_t> rank = row_morton_rank(sy.grid.nc);
   d->rows.insert(d->rows.end(), rank.begin(), rank.end());
+  const std::vector<int32_t> lrank = row_morton_rank(sy.lgrid.nc);
+  sy.lrow_off = (int32_t)d->rows.size();
+  d->rows.insert(d->rows.end(), lrank.begin(), lrank.end());
   for (int k = 0; k < in->nwalls; ++k)
     d->walls.push_back(make_wall(in->wall_basis + 9 * k, in->wall_centre + 3 * k,
                                  in->wall_half + 3 * k, in->wall_crust, 1));
@@ -976,6 +1110,10 @@ extern "C" int gdem_diff_commit(gdem_diff* d, int32_t nsteps, double dt, int32_t
   d->d_w = d->d_v + N;
   d->d_F = d->d_w + N;
   d->d_T = d->d_F + N;
+  DHIP(hipMalloc(&d->d_xref, sizeof(double4) * N));
+  DHIP(hipMalloc(&d->d_con, sizeof(int2) * N * 2 * kListCap));
+  DHIP(hipMalloc(&d->d_con_rank, sizeof(long long) * N * 2 * kListCap));
+  DHIP(hipMalloc(&d->d_con_count, sizeof(int32_t) * N));
   DHIP(hipMalloc(&d->d_ck, sizeof(double4) * N * nck * 5));
   // window of K steps of the stiffest system: K * smax force inputs
   DHIP(hipMalloc(&d->d_win, sizeof(double4) * N * (size_t)d->K * (size_t)smax * 3));
@@ -1095,6 +1233,10 @@ static int diff_launch(gdem_diff* d, int mode, const double* dtheta = nullptr,
   a.ntot = d->ntot;
   a.prop = d->d_prop;
   a.aux = d->d_aux;
+  a.xref = d->d_xref;
+  a.con = d->d_con;
+  a.con_rank = d->d_con_rank;
+  a.con_count = d->d_con_count;
   a.x0 = d->d_x0;
   a.v0 = d->d_v0;
   a.w0 = d->d_w0;
