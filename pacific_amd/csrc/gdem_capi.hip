@@ -1266,7 +1266,6 @@ static int force_launches(gdem_ctx* c, int mode, double dtv, double dtd, bool wr
     d.in_list = c->d_in_list;
     d.in_count = c->d_in_count;
     d.err = c->d_err;
-    d.nblk8 = nblk8;
     d.skin = skin ? c->skin : 0.;
     d.gap_unit = skin ? gap_unit(c) : 0.f;
     d.gate = gate;
@@ -1298,7 +1297,6 @@ static int force_launches(gdem_ctx* c, int mode, double dtv, double dtd, bool wr
     a.rec = c->d_rec;
     a.rec_count = c->d_rec_count;
     a.rec_cap = c->rec_cap;
-    a.nblk8 = nblk8;
     if (skin) {
       a.gate = gate;
       a.words = c->d_skin;

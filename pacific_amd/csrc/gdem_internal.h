@@ -233,6 +233,8 @@ struct ForceArgs {
   int32_t* in_count;  // read, then cleared for the next detection
   double4* F;  // written when non-null
   double4* T;
+  double* Fid;  // MODE_FORCE: [3 n] by particle id, written when non-null
+  double* Tid;
   int32_t* key_out;
   unsigned long long* err;
   unsigned long long* contacts;  // contact counts, one per workgroup (added to)
@@ -394,6 +396,9 @@ void launch_keys(const State& s, int32_t n, const Grid& g, const int32_t* row_ra
 // them the binning runs only when the gate says a rebuild is due; it then
 // computes the keys from src itself and clears in_count for the sweep, and
 // its first kernel does the evaluation's skin-word duties (SkinWords).
+// The binning after the count pass: b.key, b.slot and b.cnt are filled.
+void launch_sort(Bins& b, const PosSrc& src, int32_t n, const Grid& g, hipStream_t st,
+                 SkinGate gate = SkinGate{});
 void launch_binning(Bins& b, const PosSrc& src, int32_t n, const Grid& g, const int32_t* row_rank,
                     unsigned long long* err, hipStream_t st, SkinGate gate = SkinGate{},
                     SkinWords* words = nullptr, int32_t* in_count = nullptr);
@@ -401,7 +406,7 @@ void launch_binning(Bins& b, const PosSrc& src, int32_t n, const Grid& g, const 
 void launch_scan(const Bins& b, int32_t ncell, SkinGate gate, hipStream_t st);
 void launch_list_peak(const int32_t* out, const int32_t* in, int32_t n, int32_t* peak,
                       hipStream_t st);
-void launch_detect(const DetectArgs& a, hipStream_t st);
+void launch_detect(DetectArgs a, hipStream_t st);
 // With events, they record the kernel's own start and end (timing).  memory:
 // the history-model variant (a.hin / a.hout used).
 void launch_force(int mode, bool record, const ForceArgs& a, hipStream_t st,
@@ -412,7 +417,7 @@ void launch_force(int mode, bool record, const ForceArgs& a, hipStream_t st,
 void launch_wall_loads(const ForceArgs& a, double4* part, double4* out, hipStream_t st);
 // Skin lists: candidate sweep (d.gate set) or screening of the lists (writes
 // f.cmask), in one launch.
-void launch_detect_screen(const DetectArgs& d, const ForceArgs& f, hipStream_t st);
+void launch_detect_screen(DetectArgs d, const ForceArgs& f, hipStream_t st);
 // gate (skin lists): the path lengths grow and need[gate.p] is raised when
 // one passes the limit.
 void launch_move(const State& s, const double4* F, const double4* T, int32_t n, const Grid& g,

@@ -215,7 +215,7 @@ __global__ void __launch_bounds__(kBlock) k_force(ForceArgs a) {
   __syncthreads();
   if (threadIdx.x == 0) {
     unsigned long long tot = 0;
-    for (int w = 0; w < kBlock / 64; ++w) tot += sh_cnt[w];
+    for (int w = 0; w < (int)blockDim.x / 64; ++w) tot += sh_cnt[w];
     if (tot) a.contacts[blockIdx.x] += tot;  // this workgroup's slot: no atomics
   }
 }
@@ -435,12 +435,17 @@ void launch_binning(Bins& b, const PosSrc& src, int32_t n, const Grid& g, const 
   // least: the count pass also updates the skin words
   const bool gated = gate.w != nullptr;
   auto capped = [gated](int blocks) { return gated ? std::min(blocks, kGateGrid) : blocks; };
-  const int ncell = g.ncell;
   hipLaunchKernelGGL(k_count, dim3(capped(nblocks(n > 0 ? n : 1, kBlock))), dim3(kBlock), 0, st,
                      b.key, b.slot, b.cnt, n, gate, words, in_count, src, g, row_rank, err);
-  const int nb = nblocks(ncell, kScanCells);
-  hipLaunchKernelGGL(k_scan, dim3(nb), dim3(kScanBlock), 0, st, b.cnt, b.local, b.bsum, b.ticket,
-                     ncell, nb, gate);
+  launch_sort(b, src, n, g, st, gate);
+}
+
+void launch_sort(Bins& b, const PosSrc& src, int32_t n, const Grid& g, hipStream_t st,
+                 SkinGate gate) {
+  const bool gated = gate.w != nullptr;
+  auto capped = [gated](int blocks) { return gated ? std::min(blocks, kGateGrid) : blocks; };
+  const int ncell = g.ncell;
+  launch_scan(b, ncell, gate, st);
   if (n > 0)
     hipLaunchKernelGGL(k_scatter, dim3(capped(nblocks(n, kBlock))), dim3(kBlock), 0, st, b.key,
                        b.slot, b.local, b.bsum, b.perm, n, gate);
@@ -490,19 +495,35 @@ void launch_wall_loads(const ForceArgs& a, double4* part, double4* out, hipStrea
                      a.nwalls, out);
 }
 
-void launch_detect(const DetectArgs& a, hipStream_t st) {
+// Particles per workgroup of the sweep and the force kernel.  Both are bound by
+// the latency of one particle's chain of loads: below 65,536 particles (four
+// waves per CU) workgroups of one wave reach every CU.  The force kernel with
+// contact memory at 8,000: 83 us in workgroups of four waves, 70 of one; both
+// at 2,000 without: 26 + 18 and 22 + 12.5 us.
+constexpr int32_t kSmallBlocks = 65536;
+static inline int small_block(int32_t n) { return n < kSmallBlocks ? 64 : kBlock; }
+static inline int blocks8(int32_t n, int bs) { return (nblocks(n, bs) + 7) / 8 * 8; }
+
+void launch_detect(DetectArgs a, hipStream_t st) {
   if (a.n <= 0) return;
-  hipLaunchKernelGGL(k_detect, dim3(a.nblk8), dim3(kBlock), 0, st, a);
+  const int bs = small_block(a.n);
+  a.nblk8 = blocks8(a.n, bs);
+  hipLaunchKernelGGL(k_detect, dim3(a.nblk8), dim3(bs), 0, st, a);
 }
 
-void launch_detect_screen(const DetectArgs& d, const ForceArgs& f, hipStream_t st) {
+void launch_detect_screen(DetectArgs d, const ForceArgs& f, hipStream_t st) {
   if (d.n <= 0) return;
-  hipLaunchKernelGGL(k_detect_screen, dim3(d.nblk8), dim3(kBlock), 0, st, d, f);
+  const int bs = small_block(d.n);
+  d.nblk8 = blocks8(d.n, bs);
+  hipLaunchKernelGGL(k_detect_screen, dim3(d.nblk8), dim3(bs), 0, st, d, f);
 }
 
 template <int M, bool R, bool MEM>
-static void force_launch(const ForceArgs& a, hipStream_t st, hipEvent_t start, hipEvent_t stop) {
-  const dim3 grid(a.nblk8), block(kBlock);
+static void force_launch(ForceArgs a, hipStream_t st, hipEvent_t start, hipEvent_t stop) {
+  // the statistics take kBlock particles per part
+  const int bs = a.stat ? kBlock : small_block(a.n);
+  a.nblk8 = blocks8(a.n, bs);
+  const dim3 grid(a.nblk8), block(bs);
   if (start)
     hipExtLaunchKernelGGL((k_force<M, R, MEM>), grid, block, 0, st, start, stop, 0, a);
   else

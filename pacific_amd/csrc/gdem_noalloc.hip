@@ -14,6 +14,7 @@
 #include <mutex>
 
 #include "../../include/gdem.h"
+#include "gdem_binning.h"
 #include "gdem_host.h"
 #include "gdem_internal.h"
 
@@ -29,12 +30,13 @@ constexpr size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
 // Byte offsets of the buffers in the scratch array (sized for the maxima).
 struct NaLayout {
-  size_t state[2][6], F, T, key, slot, perm, pos, cnt, local, bsum, cell_start, row_rank, out_list,
+  size_t state[2][6], key, slot, perm, pos, cnt, local, bsum, cell_start, row_rank, out_list,
       out_count, in_list, in_count, models, err, contacts, total;
 };
 
 constexpr int64_t kNaScanBlocks = (kNaCells + kScanCells - 1) / kScanCells;
-constexpr int64_t kNaBlk8 = ((kNaParticles + kNaBlock - 1) / kNaBlock + 7) / 8 * 8;
+// contact slots: one per workgroup of the force kernel, 64 particles at least
+constexpr int64_t kNaBlk8 = ((kNaParticles + 63) / 64 + 7) / 8 * 8;
 
 constexpr NaLayout na_layout() {
   NaLayout L{};
@@ -48,8 +50,6 @@ constexpr NaLayout na_layout() {
     for (int a = 0; a < 5; ++a) L.state[k][a] = take(sizeof(double4) * kNaParticles);
     L.state[k][5] = take(sizeof(Aux) * kNaParticles);
   }
-  L.F = take(sizeof(double4) * kNaParticles);
-  L.T = take(sizeof(double4) * kNaParticles);
   L.key = take(sizeof(int32_t) * kNaParticles);
   L.slot = take(sizeof(int32_t) * kNaParticles);
   L.perm = take(sizeof(int32_t) * kNaParticles);
@@ -139,21 +139,34 @@ __global__ void __launch_bounds__(kNaBlock) k_na_prepare(int32_t* cnt, int ncell
 // The state copy the evaluation reads, in particle order: position and
 // radius, velocity and mass, angular velocity and equivalent-sphere radius
 // as given; identity orientation (the body-frame angular velocity is then the
-// world one); id = index, material 0, the given crust.
+// world one); id = index, material 0, the given crust.  Then the particle's
+// cell key and the count pass of the binning: a call on few particles costs
+// its launches, so what depends on the same particle alone shares one.
 __global__ void __launch_bounds__(kNaBlock) k_na_load(State s, const double4* pos_r,
                                                       const double4* vel_m,
                                                       const double4* om_req, double crust,
-                                                      int n, int32_t* in_count) {
+                                                      int n, int32_t* in_count, Bins b, Grid g,
+                                                      const int32_t* row_rank,
+                                                      unsigned long long* err) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 w = om_req[i];
-  s.pos_r[i] = pos_r[i];
-  s.vel_m[i] = vel_m[i];
-  s.om_req[i] = w;
-  s.wbf_I[i] = make_double4(w.x, w.y, w.z, 0.);
-  s.quat[i] = make_double4(0., 0., 0., 1.);
-  s.aux[i] = Aux{i, 0, crust};
-  in_count[i] = 0;
+  if (i < n) {
+    const double4 w = om_req[i], p = pos_r[i];
+    s.pos_r[i] = p;
+    s.vel_m[i] = vel_m[i];
+    s.om_req[i] = w;
+    s.wbf_I[i] = make_double4(w.x, w.y, w.z, 0.);
+    s.quat[i] = make_double4(0., 0., 0., 1.);
+    s.aux[i] = Aux{i, 0, crust};
+    in_count[i] = 0;
+    int k = key_of(g, row_rank, p);
+    if (k < 0) {
+      atomicMin(&err[kErrSim], (unsigned long long)(uint32_t)i);
+      k = 0;
+    }
+    b.key[i] = k;
+  }
+  // every lane of the wave takes part; lane i reads the key it wrote
+  count_pass(b.key, b.slot, b.cnt, n, false, nullptr, PosSrc{}, g, row_rank, err);
 }
 
 template <typename T>
@@ -201,6 +214,12 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     rc = na_scratch(cfg->device, &base);
     if (rc) break;
     const hipStream_t st = static_cast<hipStream_t>(stream);
+    // the call reads its error words back, so it cannot be captured
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive) {
+      rc = GDEM_ERR_HIP;
+      break;
+    }
     const int32_t nn = (int32_t)n;
     Bins b{};
     b.key = at<int32_t>(base, kNa.key);
@@ -218,8 +237,6 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     unsigned long long* err = at<unsigned long long>(base, kNa.err);
     unsigned long long* contacts = at<unsigned long long>(base, kNa.contacts);
     Model* model = at<Model>(base, kNa.models);
-    const int nblk = (int)((n + 255) / 256);
-    const int nblk8 = ((nblk + 7) / 8) * 8;
     const int nrows = g.nc[1] * g.nc[2];
     const int prep = (int)std::max<int64_t>(std::max<int64_t>(g.ncell, nrows), kNaBlk8);
     hipLaunchKernelGGL(k_na_prepare, dim3(std::min((prep + kNaBlock - 1) / kNaBlock, 1024)),
@@ -230,9 +247,9 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     hipLaunchKernelGGL(k_na_load, dim3((nn + kNaBlock - 1) / kNaBlock), dim3(kNaBlock), 0, st, s0,
                        reinterpret_cast<const double4*>(pos_r),
                        reinterpret_cast<const double4*>(vel_m),
-                       reinterpret_cast<const double4*>(om_req), crust, nn, in_count);
-    launch_keys(s0, nn, g, row_rank, b.key, err, st);
-    launch_binning(b, PosSrc{s0.pos_r, nullptr, s0.aux}, nn, g, row_rank, err, st);
+                       reinterpret_cast<const double4*>(om_req), crust, nn, in_count, b, g,
+                       (const int32_t*)row_rank, err);
+    launch_sort(b, PosSrc{s0.pos_r, nullptr, s0.aux}, nn, g, st);
     DetectArgs d{};
     d.pos = b.pos;
     d.margin = prefilter_margin(g, d.sizef);
@@ -248,7 +265,6 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     d.in_list = at<int2>(base, kNa.in_list);
     d.in_count = in_count;
     d.err = err;
-    d.nblk8 = nblk8;
     launch_detect(d, st);
     ForceArgs a{};
     a.in = s0;
@@ -265,21 +281,16 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     a.out_count = d.out_count;
     a.in_list = d.in_list;
     a.in_count = in_count;
-    a.F = at<double4>(base, kNa.F);
-    a.T = at<double4>(base, kNa.T);
+    a.Fid = F;
+    a.Tid = T;
     a.key_out = b.key;
     a.err = err;
     a.contacts = contacts;
-    a.nblk8 = nblk8;
     launch_force(MODE_FORCE, false, a, st);
-    // forces in particle order (the evaluation wrote them in slot order)
-    launch_unpermute(s1, a.F, a.T, nn, nullptr, nullptr, nullptr, nullptr, F, T, st);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) {
-      rc = GDEM_ERR_HIP;
-      break;
-    }
     unsigned long long h[kErrWords];
-    if (hipMemcpy(h, err, sizeof(h), hipMemcpyDeviceToHost) != hipSuccess) {
+    if (hipGetLastError() != hipSuccess ||
+        hipMemcpyAsync(h, err, sizeof(h), hipMemcpyDeviceToHost, st) != hipSuccess ||
+        hipStreamSynchronize(st) != hipSuccess) {
       rc = GDEM_ERR_HIP;
       break;
     }

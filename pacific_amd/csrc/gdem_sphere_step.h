@@ -598,6 +598,11 @@ __device__ __forceinline__ int force_particle(const ForceArgs& a, int t, double&
   a.out.quat[t] = make_double4(q.v.x, q.v.y, q.v.z, q.w);
   a.out.aux[t] = R.ax;
   a.key_out[t] = key;
+  if (MODE == MODE_FORCE && a.Fid) {
+    const size_t id = 3 * (size_t)R.ax.id;
+    a.Fid[id] = F.x; a.Fid[id + 1] = F.y; a.Fid[id + 2] = F.z;
+    a.Tid[id] = T.x; a.Tid[id + 1] = T.y; a.Tid[id + 2] = T.z;
+  }
   if (a.F) {
     a.F[t] = make_double4(F.x, F.y, F.z, 0.);
     a.T[t] = make_double4(T.x, T.y, T.z, 0.);
