@@ -169,10 +169,18 @@ __global__ void __launch_bounds__(kBlock) k_cellsort(const int32_t* local, const
 
 // ---------------------------------------------------------------- detect
 __global__ void __launch_bounds__(kBlock) k_detect(DetectArgs a) {
-  if (!a.gate.rebuild()) return;
   const int t = logical_index(a.nblk8);
   if (t >= a.n) return;
   detect_particle(a, t);
+}
+
+// Few particles: kRowLanes lanes each, kRowBlock particles per workgroup.
+constexpr int kRowBlock = 64 / kRowLanes;
+__global__ void __launch_bounds__(64) k_detect_rows(DetectArgs a) {
+  __shared__ int2 hits[kListCap * 64];
+  const int per = a.nblk8 >> 3;  // as logical_index
+  const int b = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  detect_rows(a, b * kRowBlock + threadIdx.x / kRowLanes, hits + threadIdx.x, 64);
 }
 
 // Skin lists: the candidate sweep when the lists are rebuilt (need word set),
@@ -498,17 +506,19 @@ void launch_wall_loads(const ForceArgs& a, double4* part, double4* out, hipStrea
 // Particles per workgroup of the sweep and the force kernel.  Both are bound by
 // the latency of one particle's chain of loads: below 65,536 particles (four
 // waves per CU) workgroups of one wave reach every CU.  The force kernel with
-// contact memory at 8,000: 83 us in workgroups of four waves, 70 of one; both
-// at 2,000 without: 26 + 18 and 22 + 12.5 us.
+// contact memory at 8,000: 83 us in workgroups of four waves, 70 of one; at
+// 2,000 without: 18 and 12.5 us.  Below the line the sweep without a skin takes
+// kRowLanes lanes per particle (detect_rows).
 constexpr int32_t kSmallBlocks = 65536;
 static inline int small_block(int32_t n) { return n < kSmallBlocks ? 64 : kBlock; }
 static inline int blocks8(int32_t n, int bs) { return (nblocks(n, bs) + 7) / 8 * 8; }
 
 void launch_detect(DetectArgs a, hipStream_t st) {
   if (a.n <= 0) return;
-  const int bs = small_block(a.n);
-  a.nblk8 = blocks8(a.n, bs);
-  hipLaunchKernelGGL(k_detect, dim3(a.nblk8), dim3(bs), 0, st, a);
+  const bool rows = a.n < kSmallBlocks;
+  a.nblk8 = blocks8(a.n, rows ? kRowBlock : kBlock);
+  if (rows) hipLaunchKernelGGL(k_detect_rows, dim3(a.nblk8), dim3(64), 0, st, a);
+  else hipLaunchKernelGGL(k_detect, dim3(a.nblk8), dim3(kBlock), 0, st, a);
 }
 
 void launch_detect_screen(DetectArgs d, const ForceArgs& f, hipStream_t st) {

@@ -77,41 +77,51 @@ __device__ __forceinline__ int logical_index(int nblk8) {
 // swept as 5 contiguous slot ranges: cells of a row along x are consecutive in
 // the sorted order.  det.range(beg, end, sx, sy, sz, same) is called for each
 // range with the periodic shift of the candidates' image.
+// Own row: the rest of this cell (same cell, after self), then cell i+1.
+template <class Det>
+__device__ __forceinline__ void sweep_own_row(const Grid& g, const int32_t* row_rank,
+                                              const int32_t* cs, int t, const int* ijk, Det& det) {
+  const int i = ijk[0], j = ijk[1], k = ijk[2];
+  const int rb = row_base(g, row_rank, j, k);
+  det.range(t + 1, cs[rb + i + 1], 0, 0, 0, true);
+  if (i + 1 < g.nc[0]) det.range(cs[rb + i + 1], cs[rb + i + 2], 0, 0, 0, false);
+  else if (g.periodic[0]) det.range(cs[rb], cs[rb + 1], 1, 0, 0, false);
+}
+
+// Row (j + dj, k + dk), dj and dk one of (0, 1), (1, -1), (1, 0), (1, 1):
+// cells i-1 .. i+1.
+template <class Det>
+__device__ __forceinline__ void sweep_row(const Grid& g, const int32_t* row_rank,
+                                          const int32_t* cs, const int* ijk, int dj, int dk,
+                                          Det& det) {
+  const int i = ijk[0], ni = g.nc[0];
+  const bool px = g.periodic[0] != 0;
+  int jj = ijk[1] + dj, kk = ijk[2] + dk;
+  int sy = 0, sz = 0;
+  if (jj >= g.nc[1]) {
+    if (!g.periodic[1]) return;
+    jj -= g.nc[1];
+    sy = 1;
+  }
+  if (kk < 0 || kk >= g.nc[2]) {
+    if (!g.periodic[2]) return;
+    if (kk < 0) { kk += g.nc[2]; sz = -1; }
+    else { kk -= g.nc[2]; sz = 1; }
+  }
+  const int rb = row_base(g, row_rank, jj, kk);
+  const int lo = max(i - 1, 0), hi = min(i + 1, ni - 1);
+  if (px && i - 1 < 0) det.range(cs[rb + ni - 1], cs[rb + ni], -1, sy, sz, false);
+  det.range(cs[rb + lo], cs[rb + hi + 1], 0, sy, sz, false);
+  if (px && i + 1 >= ni) det.range(cs[rb], cs[rb + 1], 1, sy, sz, false);
+}
+
 template <class Det>
 __device__ __forceinline__ void half_stencil_sweep(const Grid& g, const int32_t* row_rank,
                                                    const int32_t* cs, int t, const int* ijk,
                                                    Det& det) {
-  const int i = ijk[0], j = ijk[1], k = ijk[2];
-  const int ni = g.nc[0];
-  const bool px = g.periodic[0] != 0;
-  // own row: the rest of this cell (same cell, after self), then cell i+1
-  {
-    const int rb = row_base(g, row_rank, j, k);
-    det.range(t + 1, cs[rb + i + 1], 0, 0, 0, true);
-    if (i + 1 < ni) det.range(cs[rb + i + 1], cs[rb + i + 2], 0, 0, 0, false);
-    else if (px) det.range(cs[rb], cs[rb + 1], 1, 0, 0, false);
-  }
-  // rows (j, k+1), (j+1, k-1), (j+1, k), (j+1, k+1): cells i-1 .. i+1
+  sweep_own_row(g, row_rank, cs, t, ijk, det);
   const int drow[4][2] = {{0, 1}, {1, -1}, {1, 0}, {1, 1}};
-  for (int q = 0; q < 4; ++q) {
-    int jj = j + drow[q][0], kk = k + drow[q][1];
-    int sy = 0, sz = 0;
-    if (jj >= g.nc[1]) {
-      if (!g.periodic[1]) continue;
-      jj -= g.nc[1];
-      sy = 1;
-    }
-    if (kk < 0 || kk >= g.nc[2]) {
-      if (!g.periodic[2]) continue;
-      if (kk < 0) { kk += g.nc[2]; sz = -1; }
-      else { kk -= g.nc[2]; sz = 1; }
-    }
-    const int rb = row_base(g, row_rank, jj, kk);
-    const int lo = max(i - 1, 0), hi = min(i + 1, ni - 1);
-    if (px && i - 1 < 0) det.range(cs[rb + ni - 1], cs[rb + ni], -1, sy, sz, false);
-    det.range(cs[rb + lo], cs[rb + hi + 1], 0, sy, sz, false);
-    if (px && i + 1 >= ni) det.range(cs[rb], cs[rb + 1], 1, sy, sz, false);
-  }
+  for (int q = 0; q < 4; ++q) sweep_row(g, row_rank, cs, ijk, drow[q][0], drow[q][1], det);
 }
 
 // Reduces the per-thread statistics of a workgroup of bs threads into its
