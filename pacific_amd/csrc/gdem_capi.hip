@@ -592,6 +592,19 @@ static void update_skin(gdem_ctx* c) {
   c->graph_gen++;
 }
 
+// From candidate lists to contact lists: the sweep without a skin appends to
+// cleared incoming counts, which the lists held, and bins by the keys of the
+// present positions, which the packed step does not keep.
+static int leave_skin(gdem_ctx* c) {
+  if (c->n <= 0) return GDEM_OK;
+  HIP_TRY(hipMemsetAsync(c->d_in_count, 0, sizeof(int32_t) * (size_t)c->n, c->stream));
+  launch_keys(c->buf[c->cur], (int32_t)c->n, c->grid, c->d_row_rank, c->bins.key, c->d_err,
+              c->stream);
+  HIP_TRY(hipGetLastError());
+  c->binned = false;
+  return GDEM_OK;
+}
+
 extern "C" int gdem_set_skin(gdem_ctx* c, double skin) {
   if (!c || !(skin == skin)) return GDEM_ERR_ARG;
   HIP_TRY(hipSetDevice(c->dev));
@@ -599,7 +612,12 @@ extern "C" int gdem_set_skin(gdem_ctx* c, double skin) {
   const int rl = ensure_canon(c);
   if (rl) return rl;
   c->skin_req = skin;
+  const bool listed = c->skin > 0.;
   update_skin(c);
+  if (listed && !(c->skin > 0.)) {
+    const int rs = leave_skin(c);
+    if (rs) return rs;
+  }
   return reset_skin_words(c);  // rebuild at the next evaluation
 }
 
