@@ -129,12 +129,13 @@ struct gdem_ctx {
   PairRec* d_prec = nullptr;
   int32_t* d_path_rows = nullptr;
   StepWords* h_step = nullptr;   // pinned: progress read back after a batch of chunks
-  double chunk_yield = kChunkSteps;  // steps a chunk of the last call did on average
-  // captured chunks: [0] one rebuild offered per kChunkSteps steps, [1] one
-  // before every step
-  hipGraphExec_t chunk_exec[2] = {nullptr, nullptr};
-  double chunk_dt[2] = {0., 0.};
-  int64_t chunk_made[2] = {-1, -1};
+  ChunkPolicy chunks;
+  // captured groups of kChunkSteps steps: [k] in chunks of 2^k steps
+  struct ChunkGraph {
+    hipGraphExec_t exec = nullptr;
+    double dt = 0.;
+    int64_t made = -1;
+  } chunk_graphs[5];
   // history (memory) contact models: per-particle memory tables, one per
   // state copy; allocated once a memory model is set and particles exist
   bool has_memory = false;
@@ -439,8 +440,8 @@ extern "C" int gdem_destroy(gdem_ctx* c) {
   free_wall_loads(c);
   free_pack(c);
   (void)hipHostFree(c->h_step);
-  for (auto& g : c->chunk_exec)
-    if (g) (void)hipGraphExecDestroy(g);
+  for (auto& g : c->chunk_graphs)
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
   for (auto& e : c->ev_pool) { (void)hipEventDestroy(e.start); (void)hipEventDestroy(e.stop); }
   for (auto& row : c->graph_exec)
     for (auto& g : row)
@@ -518,6 +519,7 @@ static int alloc_particles(gdem_ctx* c, int64_t n, bool convex) {
   c->n = n;
   c->convex = convex;
   c->rmax = 0.;
+  c->chunks = ChunkPolicy{};
   c->graph_gen++;
   const size_t nn = (size_t)std::max<int64_t>(n, 1);
   if (alloc_state(c->buf[0], n) || alloc_state(c->buf[1], n)) return GDEM_ERR_HIP;
@@ -1163,21 +1165,24 @@ static int chunk_launches(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, i
   return GDEM_OK;
 }
 
-// kChunkSteps steps as one graph, captured on first use: one chunk (each =
-// false) or a chunk per step.
-static int chunk_graph(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, bool each, double dt) {
-  const int k = each ? 1 : 0;
-  hipGraphExec_t& ge = c->chunk_exec[k];
-  if (!ge || c->chunk_dt[k] != dt || c->chunk_made[k] != c->graph_gen) {
-    if (ge) {
-      HIP_TRY(hipGraphExecDestroy(ge));
-      ge = nullptr;
+// A group of kChunkSteps steps in chunks of len (a power of two), one launch
+// at a time or as a graph captured on first use.
+static int chunk_group(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, int len) {
+  int rc = GDEM_OK;
+  for (int j = 0; j < kChunkSteps && rc == GDEM_OK; j += len) rc = chunk_launches(c, a, d, len);
+  return rc;
+}
+
+static int chunk_graph(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, int len, double dt) {
+  static_assert(kChunkSteps == 16, "one graph per power of two");
+  gdem_ctx::ChunkGraph& g = c->chunk_graphs[__builtin_ctz((unsigned)len)];
+  if (!g.exec || g.dt != dt || g.made != c->graph_gen) {
+    if (g.exec) {
+      HIP_TRY(hipGraphExecDestroy(g.exec));
+      g.exec = nullptr;
     }
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int rc = GDEM_OK;
-    if (!each) rc = chunk_launches(c, a, d, kChunkSteps);
-    else
-      for (int j = 0; j < kChunkSteps && rc == GDEM_OK; ++j) rc = chunk_launches(c, a, d, 1);
+    const int rc = chunk_group(c, a, d, len);
     hipGraph_t graph = nullptr;
     const hipError_t e = hipStreamEndCapture(c->stream, &graph);
     if (rc) {
@@ -1185,21 +1190,21 @@ static int chunk_graph(gdem_ctx* c, const StepArgs& a, const DetectArgs& d, bool
       return rc;
     }
     HIP_TRY(e);
-    const hipError_t ei = hipGraphInstantiate(&ge, graph, nullptr, nullptr, 0);
+    const hipError_t ei = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
     (void)hipGraphDestroy(graph);
     HIP_TRY(ei);
-    c->chunk_dt[k] = dt;
-    c->chunk_made[k] = c->graph_gen;
+    g.dt = dt;
+    g.made = c->graph_gen;
   }
-  HIP_TRY(hipGraphLaunch(ge, c->stream));
+  HIP_TRY(hipGraphLaunch(g.exec, c->stream));
   return GDEM_OK;
 }
 
-// n steps in the packed layout after launch_move_pack.  A chunk does
-// kChunkSteps steps unless a rebuild falls into it, so the host launches the
-// chunks it expects to need, reads the progress and launches the rest; every
-// chunk does at least one step.  With the occupancy check off the call must
-// not wait for the stream: a rebuild is then offered before every step.
+// n steps in the packed layout after launch_move_pack.  A chunk does all its
+// steps unless a rebuild falls into it, so the host launches the chunks it
+// expects to need (ChunkPolicy), reads the progress and launches the rest;
+// every chunk does at least one step.  With the occupancy check off the call
+// must not wait for the stream: a rebuild is then offered before every step.
 static int packed_steps(gdem_ctx* c, int32_t n, double dt) {
   StepArgs a;
   DetectArgs d;
@@ -1209,28 +1214,34 @@ static int packed_steps(gdem_ctx* c, int32_t n, double dt) {
   if (!c->skin_adapt || c->timing) {
     for (int32_t k = 0; k < n && rc == GDEM_OK;) {
       const bool run = graph && n - k >= kChunkSteps;
-      rc = run ? chunk_graph(c, a, d, true, dt) : chunk_launches(c, a, d, 1);
+      rc = run ? chunk_graph(c, a, d, 1, dt) : chunk_launches(c, a, d, 1);
       k += run ? kChunkSteps : 1;
     }
   } else {
+    ChunkPolicy& pol = c->chunks;
+    int32_t chunks = 0, rebuilds = 0;
     for (int32_t done = 0; done < n && rc == GDEM_OK;) {
-      int32_t left = n - done;
-      if (left < kChunkSteps) {
-        rc = chunk_launches(c, a, d, left);
-      } else {
-        const int32_t chunks = std::max(1, (int32_t)((double)left / c->chunk_yield + 0.5));
-        for (int32_t k = 0; k < chunks && rc == GDEM_OK; ++k)
-          rc = graph ? chunk_graph(c, a, d, false, dt) : chunk_launches(c, a, d, kChunkSteps);
-      }
+      const bool one = step_in_one((int32_t)c->n);
+      const int32_t left = n - done;
+      const bool whole = left >= kChunkSteps;
+      const int32_t len = whole ? pol.choose(one) : pol.tail(left, one);
+      if (whole)
+        for (int32_t k = pol.groups(left, one); k > 0 && rc == GDEM_OK; --k)
+          rc = graph ? chunk_graph(c, a, d, len, dt) : chunk_group(c, a, d, len);
+      else
+        for (int32_t k = left; k > 0 && rc == GDEM_OK; k -= len)
+          rc = chunk_launches(c, a, d, std::min(k, len));
       if (rc) break;
       HIP_TRY(hipMemcpyAsync(c->h_step, c->d_step, sizeof(StepWords), hipMemcpyDeviceToHost,
                              c->stream));
       HIP_TRY(hipStreamSynchronize(c->stream));
-      done = c->h_step->slot[kChunkSteps].done;
+      const StepWords& w = *c->h_step;
+      const int32_t now = w.slot[kChunkSteps].done;
+      pol.note(now - done, whole ? (w.chunks - chunks) * len : 0, w.rebuilds - rebuilds);
+      done = now;
+      chunks = w.chunks;
+      rebuilds = w.rebuilds;
     }
-    if (rc == GDEM_OK && n >= kChunkSteps)
-      c->chunk_yield = std::min<double>(
-          kChunkSteps, std::max(1., (double)n / (double)std::max(c->h_step->chunks, 1)));
   }
   if (rc) return rc;
   for (int32_t k = 0; k < n; ++k) c->time += dt;

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gdem_chunks.h"
 #include "gdem_convex.h"
 #include "gdem_device.h"
 
@@ -83,18 +84,19 @@ struct SkinWords {
 // last one writes slot kChunkSteps, which the next chunk's rebuild kernels
 // read and copy to slot 0.  A slot holds the steps done so far, the copy the
 // next step reads, whether a rebuild is due before it, whether the last step
-// was a rebuild and whether the copy holds the world angular velocities.  A launch that finds a rebuild due (and none offered
-// right before it) or the target reached passes its slot on and does nothing
-// else, so the host may launch chunks without knowing where rebuilds fall.
-constexpr int kChunkSteps = 16;
+// was a rebuild and whether the copy holds the world angular velocities.  A
+// launch that finds a rebuild due (and none offered right before it) or the
+// target reached passes its slot on and does nothing else, so the host may
+// launch chunks without knowing where rebuilds fall.
 struct StepSlot {
   int32_t done, cur, need, rebuilt, wstored;
 };
 struct StepWords {
   StepSlot slot[kChunkSteps + 1];
-  int32_t target;  // steps of this call
-  int32_t peak;    // longest list of the last build, if near the capacity
-  int32_t chunks;  // chunks that found steps to do
+  int32_t target;    // steps of this call
+  int32_t peak;      // longest list of the last build, if near the capacity
+  int32_t chunks;    // chunks of this call that found steps to do
+  int32_t rebuilds;  // rebuilds of this call
 };
 
 // Rebuild decision: of the evaluation reading copy p (the same in every

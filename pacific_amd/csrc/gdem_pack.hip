@@ -16,13 +16,14 @@
 // pair once and stores a record that k_integ adds to both bodies.
 //
 // A rebuild of the lists (k_pk_count, k_scan, k_pk_scatter, k_pk_cellsort,
-// k_pk_sweep: the counting sort by cell and the half-stencil sweep,
-// LinkedCell.cpp:1019-1103) is launched once per chunk of kChunkSteps steps
-// and exits at once when it is not due.  When a particle's path passes the
-// skin's limit in the middle of a chunk, the remaining step kernels of that
+// k_pk_sweep, k_pk_lists: the counting sort by cell and the half-stencil sweep,
+// LinkedCell.cpp:1019-1103) is launched once per chunk of at most kChunkSteps
+// steps and exits at once when it is not due.  When a particle's path passes
+// the skin's limit in the middle of a chunk, the remaining step kernels of that
 // chunk exit without doing anything (StepWords), the next chunk starts with
 // the rebuild and continues from the step that waited: the rebuilds happen at
-// exactly the steps at which a check before every step would make them.
+// exactly the steps at which a check before every step would make them.  The
+// chunks are as long as the lists' lives make worth while (ChunkPolicy).
 //
 // The per-pair arithmetic and the order of every sum are those of the fused
 // kernel (gdem_sphere_step.h), so both give bit-identical results.  Contact
@@ -202,6 +203,7 @@ __global__ void __launch_bounds__(64) k_step_words(StepWords* w, int32_t* path_r
   w->target = 0;
   w->peak = 0;
   w->chunks = 0;
+  w->rebuilds = 0;
 }
 
 __global__ void __launch_bounds__(kPB) k_from_pack(Pack pk, PackConst k, State s, float* path_out,
@@ -246,6 +248,7 @@ __global__ void __launch_bounds__(kPB) k_pk_count(Bins b, PosSrc src0, PosSrc sr
     if (open) w->chunks += 1;
     if (rebuild) {
       words->rebuilds += 1;
+      w->rebuilds += 1;
       w->peak = 0;
     }
   }
@@ -1012,6 +1015,7 @@ __global__ void __launch_bounds__(kPB) k_move_pack(Pack pk, PackConst k, const d
     w->slot[kChunkSteps].wstored = 1;
     w->target = nsteps;
     w->chunks = 0;
+    w->rebuilds = 0;
   }
   if (i < n) {
     const double4 A4 = pk.A[i], B4 = pk.B[i], D4 = pk.D[i];
