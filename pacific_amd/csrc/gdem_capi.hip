@@ -1140,6 +1140,7 @@ static void packed_args(const gdem_ctx* c, double dt, StepArgs& a, DetectArgs& d
   d.nblk8 = (int32_t)(((c->n + 255) / 256 + 7) / 8 * 8);
   d.skin = c->skin;
   d.gap_unit = a.gap_unit;
+  d.peak = &c->d_step->peak;
   d.gate = SkinGate{nullptr, 0, a.limit, c->d_step};
 }
 

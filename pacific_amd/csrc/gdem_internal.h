@@ -167,6 +167,7 @@ struct DetectArgs {
   // sweep runs only when the gate says a rebuild is due
   double skin;
   float gap_unit;  // unit of the entries' gap bounds
+  int32_t* peak;   // longest incoming list, where it comes near the capacity (nullable)
   SkinGate gate;
 };
 

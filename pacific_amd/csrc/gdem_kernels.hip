@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(kBlock) k_cellsort(const int32_t* local, const
 __global__ void __launch_bounds__(kBlock) k_detect(DetectArgs a) {
   const int t = logical_index(a.nblk8);
   if (t >= a.n) return;
-  detect_particle(a, t);
+  detect_particle<kSweepContacts>(a, t);
 }
 
 // Few particles: kRowLanes lanes each, kRowBlock particles per workgroup.
@@ -190,7 +190,7 @@ __global__ void __launch_bounds__(kBlock) k_detect_screen(DetectArgs d, ForceArg
   const int t = logical_index(d.nblk8);
   if (t >= d.n) return;
   if (d.gate.rebuild())
-    detect_particle(d, t);
+    detect_particle<kSweepCandidates>(d, t);
   else
     screen_particle(f, t);
 }

@@ -85,9 +85,11 @@ __device__ __forceinline__ void sort_incoming(int2* l, int n, int stride) {
 // touch: its entries that touch or nearly do.  Returns the longer of the two
 // lists (the build's counts, before any cut).
 // The keys are sorted in a column of LDS (keys, one column per lane).
+// COUNTED: the incoming counts are complete.
+template <bool COUNTED>
 __device__ __forceinline__ int build_screen_list(const StepLists& l, int t, int n,
                                                  uint32_t (*keys)[kPB], int& touch) {
-  const int co = l.out_count[t], ci = l.in_count[t];
+  const int co = l.out_count[t], ci = COUNTED ? l.in_count[t] : 0;
   const int nout = min(co, kListCap), nin = l.both ? min(ci, kListCap) : 0;
   if (l.both) sort_incoming(l.in_list + t, nin, n);
   const int lane = threadIdx.x, cnt = nout + nin;
@@ -187,7 +189,7 @@ __global__ void __launch_bounds__(kPB) k_to_pack(State s, Pack pk, PackConst k0,
     len = path_in[i];
     path[i] = len;
     // without a build the lists hold nothing yet; need is set then
-    if (!l.words->slot[kChunkSteps].need) peak = build_screen_list(l, i, n, sh_keys, touch);
+    if (!l.words->slot[kChunkSteps].need) peak = build_screen_list<true>(l, i, n, sh_keys, touch);
   }
   note_peak(peak, l.words);
   wave_touch(touch, l.path_rows);
@@ -289,23 +291,38 @@ __global__ void __launch_bounds__(kPB) k_pk_cellsort(Bins b, PosSrc src0, PosSrc
 
 // The candidate sweep; grid-stride over the particles' workgroups (the grid
 // is a multiple of 8, so a workgroup stays on its XCD's range of cells).
-__global__ void __launch_bounds__(kPB) k_pk_sweep(DetectArgs d, PosSrc src0, PosSrc src1) {
+// LISTS: the screening lists hold the out entries alone, so each particle's is
+// made right after its sweep (the longest incoming list is noted by the sweep).
+// Bound by the latency of its loads: without the contact test, which candidates
+// never take, it holds 51 registers instead of 140, and seven waves share a
+// SIMD instead of three.  1M particles: sweep 173 us and lists 37 us in a kernel
+// of their own before, 149 us together.
+template <bool LISTS>
+__global__ void __launch_bounds__(kPB) k_pk_sweep(DetectArgs d, PosSrc src0, PosSrc src1,
+                                                  StepLists l) {
+  __shared__ uint32_t sh_keys[LISTS ? kListCap : 1][kPB];
   if (!d.gate.rebuild()) return;
   const PosSrc src = d.gate.sw->slot[0].cur ? src1 : src0;
   const int per = d.nblk8 >> 3;
   for (int b = blockIdx.x; b < d.nblk8; b += gridDim.x) {
     const int t = ((b & 7) * per + (b >> 3)) * kPB + threadIdx.x;
-    if (t < d.n) detect_particle(d, src, t);
+    if (t < d.n) detect_particle<kSweepCandidates>(d, src, t);
+    if (LISTS) {
+      int touch = 0;
+      note_peak(t < d.n ? build_screen_list<false>(l, t, d.n, sh_keys, touch) : 0, l.words);
+      wave_touch(touch, l.path_rows);
+    }
   }
 }
 
+// Screening lists of out and in entries: after the whole sweep.
 __global__ void __launch_bounds__(kPB) k_pk_lists(StepLists l, SkinGate gate, int n) {
   __shared__ uint32_t sh_keys[2 * kListCap][kPB];
   if (!gate.rebuild()) return;
   for (int b0 = blockIdx.x * kPB; b0 < n; b0 += gridDim.x * kPB) {
     const int t = b0 + threadIdx.x;
     int touch = 0;
-    note_peak(t < n ? build_screen_list(l, t, n, sh_keys, touch) : 0, l.words);
+    note_peak(t < n ? build_screen_list<true>(l, t, n, sh_keys, touch) : 0, l.words);
     wave_touch(touch, l.path_rows);
   }
 }
@@ -1098,8 +1115,13 @@ void launch_pack_rebuild(const Bins& b, const PosSrc& src0, const PosSrc& src1, 
   hipLaunchKernelGGL(k_pk_scatter, grid, block, 0, st, b, w, d.gate, d.n, l.path_rows);
   hipLaunchKernelGGL(k_pk_cellsort, dim3(std::min(pblocks(ncell), 1024)), block, 0, st, b, src0,
                      src1, d.gate, ncell, d.n);
-  hipLaunchKernelGGL(k_pk_sweep, dim3(std::min(d.nblk8, 2048)), block, 0, st, d, src0, src1);
-  hipLaunchKernelGGL(k_pk_lists, grid, block, 0, st, l, d.gate, d.n);
+  const dim3 sweep(std::min(d.nblk8, 2048));
+  if (l.both) {
+    hipLaunchKernelGGL(k_pk_sweep<false>, sweep, block, 0, st, d, src0, src1, l);
+    hipLaunchKernelGGL(k_pk_lists, grid, block, 0, st, l, d.gate, d.n);
+  } else {
+    hipLaunchKernelGGL(k_pk_sweep<true>, sweep, block, 0, st, d, src0, src1, l);
+  }
 }
 
 bool step_in_one(int32_t n) { return n < kStepSmall; }

@@ -21,7 +21,11 @@ struct OutList {
     a.out_list[(size_t)k * a.lstride + t] = e;
   }
 };
-template <class Out = OutList>
+// What a sweep lists: contacts, candidates (skin lists), or whichever the
+// arguments ask for.  Known at compile time the sweep of candidates holds no
+// contact test.
+enum Sweep { kSweepContacts, kSweepCandidates, kSweepAny };
+template <Sweep KIND = kSweepAny, class Out = OutList>
 struct Detector {
   const DetectArgs& a;
   Out out;
@@ -37,6 +41,10 @@ struct Detector {
   __device__ __forceinline__ Detector(const DetectArgs& a_, Out out_, const PosSrc& src_, int t_,
                                       float4 mef_)
       : a(a_), out(out_), src(src_), t(t_), mef(mef_), have_me(false), X{}, r(0.), ax{}, nout(0) {}
+
+  __device__ __forceinline__ bool candidates() const {
+    return KIND == kSweepAny ? a.skin > 0. : KIND == kSweepCandidates;
+  }
 
   // Appends partner u (entry code) to this particle's out-list and the
   // mirror entry to u's in-list; id and id2 name the two in a capacity error.
@@ -67,7 +75,7 @@ struct Detector {
     const float rsf = mef.w + p2f.w + (float)a.skin + a.margin;
     const float d2f = dxf * dxf + dyf * dyf + dzf * dzf;
     if (d2f > rsf * rsf) return;
-    if (a.skin > 0.) {
+    if (candidates()) {
       // candidate: the pre-filter alone decides (every pair with gap below
       // the skin passes it, and the few within the margin beyond); the
       // contact test of every step is made on the candidates with the same
@@ -139,6 +147,7 @@ struct Detector {
               make_int2(t, mirror_code(code) | (e << 7) | (int)((uint32_t)code & kGapMask));
         else
           atomicMin(&a.err[kErrCapacity], (unsigned long long)(uint32_t)a.ids[u]);
+        if (a.peak && kin[k] >= kListCap - kListHeadroom) atomicMax(a.peak, kin[k] + 1);
       }
     }
   }
@@ -157,20 +166,22 @@ struct Detector {
 
 // Detection sweep of one particle (storage slot t of the sorted order), with
 // positions from src.
+template <Sweep KIND = kSweepAny>
 __device__ __forceinline__ int detect_particle(const DetectArgs& a, const PosSrc& src, int t) {
   // the cell index comes from the full-precision position, as in the binning
   const double4 me = src.pos(a.perm[t]);
   int ijk[3];
   clamped_cell(a.grid, mk(me.x, me.y, me.z), ijk);
-  Detector<> det(a, OutList{a, t}, src, t, a.pos[t]);
+  Detector<KIND> det(a, OutList{a, t}, src, t, a.pos[t]);
   half_stencil_sweep(a.grid, a.row_rank, a.cell_start, t, ijk, det);
-  if (a.skin > 0.) det.link();
+  if (det.candidates()) det.link();
   a.out_count[t] = det.nout;
   return det.nout;
 }
 
+template <Sweep KIND = kSweepAny>
 __device__ __forceinline__ void detect_particle(const DetectArgs& a, int t) {
-  detect_particle(a, PosSrc{a.in.pos_r, nullptr, a.in.aux}, t);
+  detect_particle<KIND>(a, PosSrc{a.in.pos_r, nullptr, a.in.aux}, t);
 }
 
 // The same sweep for contact lists (no skin) by kRowLanes lanes of a wave, the
@@ -194,7 +205,7 @@ __device__ __forceinline__ void detect_rows(const DetectArgs& a, int t, int2* hi
     const double4 me = src.pos(a.perm[t]);
     int ijk[3];
     clamped_cell(a.grid, mk(me.x, me.y, me.z), ijk);
-    Detector<OutLds> det(a, OutLds{hits, stride}, src, t, a.pos[t]);
+    Detector<kSweepContacts, OutLds> det(a, OutLds{hits, stride}, src, t, a.pos[t]);
     if (lane == 0) sweep_own_row(a.grid, a.row_rank, a.cell_start, t, ijk, det);
     else sweep_row(a.grid, a.row_rank, a.cell_start, ijk, lane > 1, lane == 1 ? 1 : lane - 3, det);
     nout = det.nout;

@@ -3,6 +3,8 @@ to zero, and the halving that ends there): the sweep without a skin starts from
 empty incoming lists and from the keys of the present positions, so the forces,
 the contacts and the steps after it are those of a new context without a skin.
 
+The last test has lists grow long within the packed steps: the rebuild notes it.
+
 Bars: the two contexts hold the particles in different orders, so a particle's
 contacts (at most 24 and the walls) are summed in another order: 2 * 30 * 2^-53
 = 7e-15 of the sum of their magnitudes, stated as 1e-13.  After 20 further
@@ -84,23 +86,32 @@ def test_skin_switched_off_after_lists_were_built(n, periodic, recording):
         b.close()
 
 
-def _burdock(m=22):
-    """A sphere of 1 mm that touches m small ones, all within one octant past
-    the corner of its cell: each is detected by the large one."""
+def _burdock(gap=-1.0e-6, side=1.0, speed=0.0, m=22, filler=0):
+    """A sphere of 1 mm and m small ones around it at that gap, approaching at
+    that speed, all within one octant past a corner of its cell: each is
+    detected by the large one (side 1) or detects it (side -1).  filler: that
+    many small spheres at rest elsewhere, apart from each other."""
     k = np.arange(10 * m) + 0.5
     phi, z = np.pi * (1.0 + 5.0 ** 0.5) * k, 1.0 - 2.0 * k / (10 * m)
     rho = np.sqrt(1.0 - z * z)
     d = np.stack([rho * np.cos(phi), rho * np.sin(phi), z], 1)
-    d = d[(d > 0.05).all(1)][:m]
-    r = np.concatenate([[1.0e-3], np.full(len(d), 0.1e-3)])
+    d = side * d[(d > 0.05).all(1)][:m]
     wl = workloads.periodic_hooke(2000)
-    edge = 3.0e-3
-    c = np.full(3, 2.0 * edge - 1.0e-6)
-    x = np.concatenate([c[None], c + d * (1.1e-3 - 1.0e-6)])
+    edge, k = 3.0e-3, int(np.ceil(filler ** (1.0 / 3.0)))
+    c = np.full(3, 2.0 * edge - side * 1.0e-6)
+    x = np.concatenate([c[None], c + d * (1.1e-3 + gap)])
     v = np.random.default_rng(4).normal(0.0, 0.01, x.shape)
+    if speed:
+        v = np.concatenate([np.zeros((1, 3)), -d * speed])
+    if filler:
+        at = np.arange(filler)
+        x = np.concatenate([x, 4.0 * edge + 1.5e-3 * np.stack([at // (k * k), at // k % k, at % k], 1)])
+        v = np.concatenate([v, np.zeros((filler, 3))])
+    r = np.concatenate([[1.0e-3], np.full(len(x) - 1, 0.1e-3)])
     # soft contacts: a small sphere stays on the large one for some 200 steps
-    wl.update(origin=(0.0,) * 3, size=(4.0 * edge,) * 3, cell_size=edge, dt=1.0e-7, walls=[],
-              periodic=(0, 0, 0), gravity=(0.0,) * 3, particles=workloads._particles(x, v, r),
+    wl.update(origin=(0.0,) * 3, size=(8.0 * edge + 1.5e-3 * k,) * 3, cell_size=edge, dt=1.0e-7,
+              walls=[], periodic=(0, 0, 0), gravity=(0.0,) * 3,
+              particles=workloads._particles(x, v, r),
               models=[(0, 0, gdem.MODEL_HOOKE, (2.0e2, 0.9, -1.0, 0.5, 0.0))])
     return wl, len(r)
 
@@ -121,3 +132,28 @@ def test_halving_that_ends_without_a_skin():
     _same_steps(a, b, wl)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("filler", [0, 524300])   # one kernel per step, two
+@pytest.mark.parametrize("side", [1.0, -1.0])     # long out list, long in list
+def test_rebuild_of_the_packed_step_notes_long_lists(filler, side):
+    """The lists of the first evaluation are short; those of a rebuild within
+    the packed steps come near the capacity and halve the skin."""
+    print(f"[case] halving on a packed rebuild, {filler} others, side {side}", flush=True)
+    wl, n = _burdock(gap=0.24e-3, side=side, speed=2.0, filler=filler)
+    wl["dt"] = 1.0e-6
+    a = gdem.build_system(wl)
+    skin = a.get_skin()[0]
+    assert 0.19e-3 < skin < 0.21e-3
+    a.step(20, wl["dt"])
+    occ = a.list_occupancy()
+    assert occ["skin_halvings"] == 0 and a.get_skin()[1] == 1, occ
+    a.step(60, wl["dt"])
+    occ = a.list_occupancy()
+    assert occ["skin_halvings"] == 1 and occ["peak"] == 22, occ
+    assert a.get_skin()[0] == 0.5 * skin
+    a.step(20, wl["dt"])
+    st = a.get_state()
+    want = wl["particles"]["x"] + 100 * wl["dt"] * wl["particles"]["v"]
+    assert np.abs(st["x"] - want).max() <= 1e-12   # free flight, 100 sums of 1e-6 m
+    a.close()
