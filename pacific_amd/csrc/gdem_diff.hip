@@ -381,6 +381,7 @@ struct DiffRunner {
       }
       if (threadIdx.x == 0) {
         DetectArgs& d = *sd;
+        d = DetectArgs{};  // fields not set below are null / zero
         d.pos = pos;
         d.sizef[0] = sy.sizef[0]; d.sizef[1] = sy.sizef[1]; d.sizef[2] = sy.sizef[2];
         d.margin = sy.margin;
@@ -398,10 +399,8 @@ struct DiffRunner {
         d.in_list = a.in_list + (size_t)sy.off * kListCap;
         d.in_count = a.in_count + sy.off;
         d.err = err();
-        d.nblk8 = 0;
         d.skin = skin;
         d.gap_unit = 1.f;  // the entries' gap bounds are not used
-        d.gate = SkinGate{};
         smem[1] = 0;
       }
       __syncthreads();
