@@ -56,9 +56,9 @@ __device__ __forceinline__ Orient load_orient(const CState& c, int s) {
 // each other's narrow phase.
 //
 // kSweepLanes lanes sweep one particle together (eight for few particles, two
-// for many): each takes every kSweepLanes-th slot of a range and the kept candidates are appended in slot
-// order (ballot over the particle's lanes), so the lists are those of a
-// serial sweep.  The sweep is a chain of loads and tests, about 100 slots per
+// for many): each takes every kSweepLanes-th slot of a range and the kept
+// candidates are appended in slot order (ballot over the particle's lanes), so
+// the lists are those of a serial sweep.  The sweep is a chain of loads and tests, about 100 slots per
 // particle: with one lane per particle it took 35 us at 3,000 particles as at
 // 40,000.
 template <int kSweepLanes>
@@ -356,9 +356,20 @@ __device__ __forceinline__ void narrow_phase(const CGjkArgs& a, int item) {
 // spheres overlap, the bodies do not) to the queue of the narrow phase; one
 // integer atomic per workgroup.  With statistics on every candidate is
 // evaluated: its GJK iterations count.  A queue of at most kFilterFrom
-// candidates is left as it is: its waves run side by side, and the filter's
-// 20 us would come on top of the slowest one.
-constexpr int kFilterFrom = 32768;
+// candidates is left as it is: the GJK runs one wave per SIMD, 1,024 of 64
+// lanes on the chip, and takes as long as its slowest wave, so within one round
+// of waves the filter's 20 us come on top.  Steps of n bodies at solid fraction
+// phi, filter off and on, us (Johnson; signed volumes):
+//   n, phi        candidates   Johnson    signed volumes
+//   12,000, 0.20      34,103   150, 171   162, 180
+//   30,000, 0.10      35,062   160, 183   173, 193
+//   20,000, 0.20      56,321   159, 182   172, 193
+//   16,000, 0.25      59,669   159, 182   174, 195
+//   25,000, 0.20      70,189   204, 188   226, 198
+//   20,000, 0.25      74,212   215, 186   235, 197
+//   40,000, 0.20     111,805   234, 195   260, 208
+//   200,000, 0.25    722,545   916, 367   1,052, 395
+constexpr int kFilterFrom = 65536;
 __global__ void __launch_bounds__(kCBlock) k_cfilter(CGjkArgs a) {
   __shared__ int sh_wave[kCBlock / 64], sh_base;
   const int nw = *a.nwork;
@@ -386,7 +397,7 @@ __global__ void __launch_bounds__(kCBlock) k_cfilter(CGjkArgs a) {
 
 // Workgroups of one wave: the GJK holds all registers of a SIMD and a wave is
 // as slow as its slowest lane, so waves are spread over the compute units one
-// by one.  40,000 bodies at solid fraction 0.20 (160,000 candidates): 169 us
+// by one.  40,000 bodies at solid fraction 0.20 (112,000 candidates): 169 us
 // per launch over the whole queue in workgroups of four waves; filter 23 us
 // and 108 us for what it leaves.
 constexpr int kGjkBlock = 64;
@@ -734,7 +745,10 @@ static inline int cblocks(int n) { return (n + kCBlock - 1) / kCBlock; }
 
 void launch_cdetect(const CDetectArgs& a, hipStream_t st) {
   if (a.n <= 0) return;
-  const bool few = a.n < 32768;
+  // us per step with 8 and 2 lanes at solid fraction 0.20: 3,000 bodies 135 and
+  // 143, 16,000 154 and 159, 25,000 203 and 203, 40,000 199 and 195; at 0.10
+  // 30,000 160 and 155; at 0.25 200,000 417 and 365
+  const bool few = a.n < 24576;
   const int p = kCBlock / (few ? 8 : 2);
   const int nblk8 = ((a.n + p - 1) / p + 7) / 8 * 8;
   if (few) hipLaunchKernelGGL(k_cdetect<8>, dim3(nblk8), dim3(kCBlock), 0, st, a, nblk8);

@@ -1,25 +1,35 @@
-"""Candidate filter and cooperative sweep of the convex step: a packing whose
-queue is long enough for the filter, where contact statistics (which switch
-the filter off) must not change a bit of the state, and the candidate lists of
-both sweep widths against the serial ones through the contact records."""
+"""Candidate filter and cooperative sweep of the convex step, in packings whose
+queue is longer than one round of narrow-phase waves (65,536 candidates), so
+that the filter runs.  Contact statistics switch the filter off and count the
+candidates: they must not change a bit of the state.  Contacts and forces of
+both sweep widths against the CPU oracle's, whose candidates come from its own
+linked cells: a candidate the sweep lost or the filter dropped would be missing.
+Bars: pairs exact, forces and torques within 1e-12 of the per-particle scale, as
+in the parity tests."""
 import numpy as np
 import pytest
 
+from gdem_testutil import force_scales, normwise_ok, pair_set
 from pacific_amd import gdem, workloads
 
 pytestmark = pytest.mark.gpu
 
 
-# 12,000 bodies: eight lanes per particle; 33,000: two
-@pytest.mark.parametrize("n,narrow", [(12000, "GJK"), (12000, "GJK_SV"), (33000, "GJK")])
-def test_filter_drops_no_contact(n, narrow):
+# 24,000 bodies: eight lanes per particle; 33,000: two
+@pytest.mark.parametrize("n,phi,narrow", [(24000, 0.22, "GJK"), (24000, 0.22, "GJK_SV"),
+                                          (33000, 0.20, "GJK")])
+def test_filter_drops_no_contact(oracle_mod, n, phi, narrow):
     print(f"[case] convex filter, {n} bodies, {narrow}", flush=True)
-    wl = workloads.convex_box(n, seed=5, phi=0.20, height=0.05, overlap=2.0e-5, sigma_v=0.3)
+    wl = workloads.convex_box(n, seed=5, phi=phi, height=0.05, overlap=2.0e-5, sigma_v=0.3)
     wl["narrow_phase"] = narrow
     out = []
     for stats in (False, True):
         s = gdem.build_system(wl)
         s.set_contact_stats(stats)
+        if stats:
+            s.prime()
+            # every candidate reports its iterations once
+            assert s.contact_stats()["gjk_reports"] > 65536
         s.step(60, wl["dt"])
         out.append((s.get_state(), s.get_basis(), s.counters()["contacts"]))
         s.close()
@@ -27,3 +37,28 @@ def test_filter_drops_no_contact(n, narrow):
     assert np.array_equal(out[0][1], out[1][1])
     for k in ("x", "v", "w", "q", "F", "T"):
         assert np.array_equal(out[0][0][k], out[1][0][k]), k
+
+
+@pytest.mark.parametrize("n,phi,narrow", [(24000, 0.22, "GJK"), (24000, 0.22, "GJK_SV"),
+                                          (33000, 0.20, "GJK")])
+def test_contacts_equal_the_oracles(oracle_mod, n, phi, narrow):
+    print(f"[case] convex filter vs oracle, {n} bodies, {narrow}", flush=True)
+    wl = workloads.convex_box(n, seed=6, phi=phi, height=0.05, overlap=2.0e-5, sigma_v=0.3)
+    wl["narrow_phase"] = narrow
+    orc = oracle_mod.ConvexOracle(wl, log_capacity=20 * n)
+    orc.prime()
+    oc, os_ = orc.contacts(), orc.state()
+    s = gdem.build_system(wl)
+    s.set_contact_recording(32)
+    s.prime()
+    gc, gs = s.get_contacts(), s.get_state()
+    s.close()
+    assert len(gc["id0"]) == len(oc["id0"]) > 1000
+    assert pair_set(gc) == pair_set(oc)
+    vols = np.array([orc.shape_info(k)[0] for k in range(len(wl["shapes"]))])
+    p = wl["particles"]
+    weight = (p["density"] * vols[p["shape"]])[:, None] * np.array(wl["gravity"])[None, :]
+    sf, st = force_scales(n, oc, p["x"], weight)
+    for got, want, scale in ((gs["F"], os_["F"], sf), (gs["T"], os_["T"], st)):
+        ok, err, bad = normwise_ok(got, want, scale, 1e-12)
+        assert ok, (np.nonzero(bad)[0][:5], err[bad][:5])
