@@ -503,19 +503,24 @@ void launch_wall_loads(const ForceArgs& a, double4* part, double4* out, hipStrea
                      a.nwalls, out);
 }
 
-// Particles per workgroup of the sweep and the force kernel.  Both are bound by
-// the latency of one particle's chain of loads: below 65,536 particles (four
-// waves per CU) workgroups of one wave reach every CU.  The force kernel with
-// contact memory at 8,000: 83 us in workgroups of four waves, 70 of one; at
-// 2,000 without: 18 and 12.5 us.  Below the line the sweep without a skin takes
-// kRowLanes lanes per particle (detect_rows).
+// Particles per workgroup of the screening and the force kernel.  Both are bound
+// by the latency of one particle's chain of loads: below 65,536 particles (four
+// waves per CU) workgroups of one wave reach every CU.  A bed with contact
+// memory, us per step in workgroups of four waves and of one: 8,000 particles 93
+// and 77, 30,000 97 and 93, 60,000 97 and 96, 80,000 115 and 115.
 constexpr int32_t kSmallBlocks = 65536;
+// Below this line the sweep without a skin takes kRowLanes lanes per particle
+// (detect_rows).  us per step with one lane and with kRowLanes: a gas of 20,000
+// 60 and 48, of 48,000 64 and 59, of 64,000 65 and 65; a touching bed of 20,000
+// 104 and 86, of 40,000 107 and 108, of 48,000 116 and 115, of 56,000 110 and
+// 126 (7,000 waves of the rows' sweep, of which 4,096 are resident).
+constexpr int32_t kRowsBelow = 49152;
 static inline int small_block(int32_t n) { return n < kSmallBlocks ? 64 : kBlock; }
 static inline int blocks8(int32_t n, int bs) { return (nblocks(n, bs) + 7) / 8 * 8; }
 
 void launch_detect(DetectArgs a, hipStream_t st) {
   if (a.n <= 0) return;
-  const bool rows = a.n < kSmallBlocks;
+  const bool rows = a.n < kRowsBelow;
   a.nblk8 = blocks8(a.n, rows ? kRowBlock : kBlock);
   if (rows) hipLaunchKernelGGL(k_detect_rows, dim3(a.nblk8), dim3(64), 0, st, a);
   else hipLaunchKernelGGL(k_detect, dim3(a.nblk8), dim3(kBlock), 0, st, a);

@@ -50,9 +50,10 @@ def test_noalloc_forces_equal_the_contexts(n):
 
 
 @pytest.mark.parametrize("n,periodic", [(2, False), (64, True), (65, False), (1000, True),
-                                        (4097, True), (4097, False)])
+                                        (4097, True), (4097, False), (49151, True),
+                                        (49152, True)])
 def test_row_sweep_equals_serial_sweep(n, periodic):
-    """One lane per row of the half stencil (a context below 65,536 particles
+    """One lane per row of the half stencil (a context below 49,152 particles
     without a skin) and one lane per particle (a batch) list the same contacts
     in the same order: bit-identical sums."""
     print(f"[case] row sweep vs serial sweep, {n} spheres, periodic {periodic}", flush=True)
