@@ -567,8 +567,7 @@ const char* gdem_version(void);
 /* ------------------------------------------------------------------------
  * One force evaluation of a sphere system that allocates no device memory.
  * No counterpart in the reference: it is for callers that cannot allocate
- * (code under HIP graph capture, tight serving loops, harnesses that forbid
- * hipMalloc).  It evaluates what gdem_prime / gdem_compute_forces evaluate
+ * (tight serving loops, harnesses that forbid hipMalloc).  It evaluates what gdem_prime / gdem_compute_forces evaluate
  * on a context holding the same particles (material 0, one contact model,
  * no walls): binning, detection, Hooke/Hertz contact forces and torques, and
  * the weight.  All of its buffers live in one static device array of the
@@ -586,8 +585,11 @@ const char* gdem_version(void);
  * Returns GDEM_ERR_CAPACITY when n, the cell count or the row count (cells
  * along y times cells along z) exceeds the maxima below, or when a particle
  * detects or receives more contacts than a list holds; CONTACT and
- * SIMULATION as gdem_last_error describes them.  Calls on one device share
- * the static array: calls that overlap in time on one device race. */
+ * SIMULATION as gdem_last_error describes them; GDEM_ERR_HIP, with nothing
+ * launched and the capture as it was, on a stream that is being captured
+ * (the call waits for the stream and reads its error words).  Calls on one
+ * device share the static array: calls that overlap in time on one device
+ * race. */
 #define GDEM_NOALLOC_MAX_PARTICLES 32768
 #define GDEM_NOALLOC_MAX_CELLS (1 << 19)
 #define GDEM_NOALLOC_MAX_ROWS 16384

@@ -205,6 +205,12 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     return GDEM_ERR_CAPACITY;
   if (err_ids) err_ids[0] = err_ids[1] = -1;
   if (n == 0) return GDEM_OK;
+  // the call reads its error words back, so it cannot be captured: refused
+  // before anything that could end the caller's capture
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive)
+    return GDEM_ERR_HIP;
   int prev = 0;
   if (hipGetDevice(&prev) != hipSuccess) return GDEM_ERR_HIP;
   if (hipSetDevice(cfg->device) != hipSuccess) return GDEM_ERR_HIP;
@@ -213,13 +219,6 @@ extern "C" int gdem_sphere_forces_noalloc(const gdem_config* cfg, int32_t kind,
     unsigned char* base = nullptr;
     rc = na_scratch(cfg->device, &base);
     if (rc) break;
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    // the call reads its error words back, so it cannot be captured
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive) {
-      rc = GDEM_ERR_HIP;
-      break;
-    }
     const int32_t nn = (int32_t)n;
     Bins b{};
     b.key = at<int32_t>(base, kNa.key);
