@@ -368,7 +368,11 @@ int gdem_get_skin(gdem_ctx* ctx, double* skin, int64_t* rebuilds);
    (switching the lists off below 0.05 r_max) and rebuilds at the next
    evaluation, so a packing that densifies keeps running; the results do not
    depend on the skin.  The check synchronises the context's stream.
-   gdem_set_skin_adapt(ctx, 0) switches it off (on by default).
+   gdem_set_skin_adapt(ctx, 0) switches it off (on by default): gdem_step then
+   does not wait for the stream, and offers a rebuild before every step (seven
+   launches per step instead of about one and a half: 21 us per step of 1,000
+   spheres instead of 13, 30 of 100,000 instead of 21, 119 of 1,000,000 instead
+   of 105 on MI355X).
    gdem_get_list_occupancy gives the longest list of the last build (skin
    lists: candidates within the skin; otherwise the outgoing contacts of the
    last evaluation; convex: circumscribed-sphere candidates), the capacity and
@@ -518,7 +522,7 @@ int gdem_last_error(gdem_ctx* ctx, int32_t* code, int32_t* id0, int32_t* id1);
    the force kernel in ms when timing is on (events on the context's stream).
    In the packed layout of gdem_step (spheres with skin lists and memoryless
    models) the force kernel is the step kernel, which evaluates the contacts
-   and applies the leap-frog tail; beyond 524,288 particles the integrator
+   and applies the leap-frog tail; from 524,288 particles on the integrator
    kernel, which sums each particle's contact records. */
 int gdem_set_kernel_timing(gdem_ctx* ctx, int32_t on);
 int gdem_get_counters(gdem_ctx* ctx, int64_t* force_evals, int64_t* contacts,
@@ -553,7 +557,7 @@ int gdem_get_contact_stats(gdem_ctx* ctx, double* out);
 
 /* Event-timed totals (ms) and launch counts of two kernels since the last
    reset: [0] the force kernel (as gdem_get_counters), [1] the pair kernel of
-   the packed layout beyond 524,288 particles (screening and evaluation of
+   the packed layout from 524,288 particles on (screening and evaluation of
    each candidate pair once; 0 launches below).  No reference counterpart: the
    reference's phase timers (Grains.cpp:246-258) time whole phases on the CPU. */
 int gdem_get_kernel_times(gdem_ctx* ctx, double* ms, int64_t* launches);

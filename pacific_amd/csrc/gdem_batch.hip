@@ -147,8 +147,10 @@ struct BatchRunner {
   // no particle changed cell since the last sort the order stands as it is
   // (the sort is stable), and with it the cell starts: a time step is a small
   // part of a cell's crossing time, the more so in a stiff system's substeps,
-  // which are the longest chains of a launch (512 systems of 64 to 2,048, 200
-  // steps and their states: 131 ms sorting every time, 116 ms so).
+  // which are the longest chains of a launch.  512 systems of 64 to 2,048, 200
+  // steps: 83 to 95 ms sorting every time, 75 to 85 so (and 29 ms to read their
+  // states); fast enough that some particle always changes cell, 100 steps: 54
+  // and 52 ms.
   __device__ __forceinline__ void bin(const State& cur) {
     const int n = sy.n, nc = sy.grid.ncell;
     int32_t* key = a.key + sy.off;

@@ -333,8 +333,9 @@ static StepLists step_lists(const gdem_ctx* c) {
                    step_in_one((int32_t)c->n), c->d_step, c->d_path_rows};
 }
 
-// Buffers of the packed layout for the current particle count (allocated on
-// first use: about 0.8 KB per particle, half of it the screening lists).
+// Buffers of the packed layout for the current particle count, allocated on
+// first use: about 0.8 KB per particle, half of it the screening lists; from
+// kStepSmall particles on 2.3 KB, most of it the pair records.
 static int alloc_pack(gdem_ctx* c) {
   if (c->pk[0].A) return GDEM_OK;
   const size_t n = (size_t)std::max<int64_t>(c->n, 1);
@@ -1011,7 +1012,6 @@ static void launch_convex_step(gdem_ctx* c, int mode, double dtv, double dtd, bo
   d.walls = c->d_walls;
   d.nwalls = c->nwalls;
   d.err = c->d_err;
-  d.nblk8 = nblk8;
   CGjkArgs g{};
   g.in = c->buf[c->cur];
   g.cin = c->cbuf[c->cur];

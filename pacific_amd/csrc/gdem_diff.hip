@@ -216,8 +216,10 @@ struct DiffRunner {
   // overflow a list hold the contacts alone from then on, as they do where the
   // cells leave no room for a skin.  Binning and sweeping at every evaluation
   // took half of a gradient, serial phases of few memory accesses each: 512
-  // systems of 1,000 over 400 steps 672 ms with them, 494 ms so; 12 of 250
-  // over 60 steps 21.7 and 13.9 ms.  first: the first evaluation of a launch.
+  // systems of 1,000 over 400 steps 648 ms with them, 479 ms so; 12 of 250
+  // over 60 steps 18.6 and 11.8 ms.  Without room for a skin the contacts are
+  // tested twice (256 periodic cubes of 27 in three cells: 10.7 and 11.7 ms).
+  // first: the first evaluation of a launch.
   __device__ __forceinline__ void lists(bool first = false) {
     const int n = sy.n;
     if (threadIdx.x == 0) smem[1] = first || !(skin > 0.) ? 1 : 0;

@@ -310,7 +310,6 @@ struct CDetectArgs {
   const Wall* walls;
   int32_t nwalls;
   unsigned long long* err;
-  int32_t nblk8;
 };
 
 struct CGjkArgs {

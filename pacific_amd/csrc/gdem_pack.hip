@@ -1,8 +1,8 @@
 // gdem_pack.hip -- the sphere step in the packed layout (skin candidate
 // lists, memoryless contact models).
 //
-// A step that keeps its lists is one kernel up to kStepSmall particles
-// (k_step) and two beyond (k_pairs, k_integ).  Candidates are screened, the
+// A step that keeps its lists is one kernel below kStepSmall particles
+// (k_step) and two from there on (k_pairs, k_integ).  Candidates are screened, the
 // pairs that may touch are gathered into a queue in LDS and evaluated one per
 // lane with the reference's body order (RigidBodyWithCrust.cpp:596-640,
 // HookeContactForceModel.cpp:44-114 / HertzContactForceModel.cpp:46-114), and
@@ -31,15 +31,18 @@
 // gdem_step runs the canonical layout.
 //
 // Bound: below some 100,000 particles the step is one chain of dependent
-// loads and FP64 operations (about 12 us) and launches; six launches per step
-// (screening, contacts, integrator and three rebuild kernels that exit) were
-// 44 to 62 us, one launch is 15 (1,000 particles in a box), 26 (a packing of
-// 30,000) and 21.5 us (a gas of 100,000).  Many particles stream the state
-// (about 250 B each) through k_integ, and both partners' evaluations in one
-// kernel no longer hide behind it: at 1M in a gas k_step takes 125 us a step,
-// k_pairs and k_integ 113 (three kernels before: 125); at 400,000 k_step takes
-// 58 and the two 61, and in a packing of 500,000 190 to 215 against 220: the
-// line lies at kStepSmall.
+// loads and FP64 operations (about 12 us) and launches.  us per step of a call
+// (gdem_step alone), with the six launches per step of before (screening,
+// contacts, integrator and three rebuild kernels that exit) and now: 1,000
+// particles in a box 26 and 15, a touching bed of 30,000 54 to 59 and 26, a gas
+// of 100,000 40 and 21.  Many particles stream the state (about 250 B each)
+// through k_integ, and both partners' evaluations in one kernel no longer hide
+// behind it: at 1M in a gas k_step takes 125 us a step, k_pairs and k_integ 103
+// to 109 (six launches 118 to 122); at 400,000 k_step takes 58 and the two 61,
+// and in a packing of 500,000 190 to 215 against 220: the line lies at
+// kStepSmall.  With the occupancy check off (gdem_set_skin_adapt) a rebuild is
+// offered before every step, seven launches: 21 us at 1,000, 30 at 100,000, 119
+// at 1M (22, 40 and 124 before).
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -121,8 +124,8 @@ __device__ __forceinline__ void note_peak(int peak, StepWords* w) {
 }
 
 // Counter `seg` of row j.  Each counter has a cache line of its own: atomics
-// on one line are served one after another (64 counters in two lines cost
-// k_stream 100 us at 1M particles, spread over 64 lines about 2 us).
+// on one line are served one after another (64 counters in two lines cost an
+// integrating kernel 100 us at 1M particles, spread over 64 lines about 2 us).
 __device__ __forceinline__ int32_t* row_word(int32_t* rows, int j, int seg) {
   return rows + ((size_t)j * kRowSegs + seg) * kRowPad;
 }
@@ -660,10 +663,11 @@ struct ContactLds {
 
 // Force and torque of the contacts of a workgroup's particles: lane k < PP
 // brings particle t (masks cm, wm of the candidates and walls that may touch;
-// lanes without a particle bring none) and gets its sums added to F and T.  The pairs are queued in LDS, evaluated one per
-// lane in rounds of BS, and each particle adds its own in queue order:
-// candidates in the order of summation, then walls.  nc counts the contacts,
-// each pair at its out entry.  Every lane of the workgroup calls.
+// lanes without a particle bring none) and gets its sums added to F and T.
+// The pairs are queued in LDS, evaluated one per lane in rounds of BS, and each
+// particle adds its own in queue order: candidates in the order of summation,
+// then walls.  nc counts the contacts, each pair at its out entry.  Every lane
+// of the workgroup calls.
 template <int BS, bool WALLS>
 __device__ __forceinline__ void gather_contacts(const StepArgs& a, const StepView& vw,
                                                 ContactLds<BS>& sh, int t,
